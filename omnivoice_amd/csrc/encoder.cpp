@@ -11,10 +11,8 @@
 // is a convolution on the fp32 matrix cores (codec_kernels.hip):
 //  * a linear layer is a one-tap convolution;
 //  * a strided, long or grouped convolution runs over im2col columns;
-//  * attention runs per head as two batched one-tap convolutions: the
-//    transposed scores S^T[key][query] = K_h^T Q_h (K_h as the weights), a
-//    softmax down each column, and the context O_h = V_h P^T (V^T as the
-//    weights, P^T as the input);
+//  * attention is one kernel per layer over the heads' [dims][steps]
+//    projections (encoder_kernels.hip);
 //  * GELU, ELU and Snake are applied by the epilogue of the producing
 //    convolution, residual additions by its accumulation.
 // The mean of HuBERT's states is summed in double by the LayerNorm that
@@ -186,8 +184,9 @@ class EncoderEngine {
   Dense ac_out_, fc_;
   std::vector<std::unique_ptr<Stage>> stages_;
   // work buffers
-  DeviceBuffer<float> samples_, wave_, fa_, fb_, cols_, tmp_, h_, qkv_, scores_, vt_, ctx_, ff_;
+  DeviceBuffer<float> samples_, wave_, fa_, fb_, cols_, tmp_, h_, qkv_, ctx_, ff_;
   DeviceBuffer<double> sum_;
+  DeviceBuffer<std::uint16_t> heads_;  // the attention's operands
   // Split-K workspace of the thin GEMMs (HuBERT at short lengths, the
   // semantic encoder, the quantizer's projections).
   DeviceBuffer<float> partial_;
@@ -510,8 +509,9 @@ void EncoderEngine::Reserve(const Plan& p) {
   grow(tmp_, hid);
   grow(h_, W * T);
   grow(qkv_, 3 * W * T);
-  grow(scores_, scores);
-  grow(vt_, W * T);
+  grow(heads_, static_cast<int64_t>(PackedHeadsElements(
+                   static_cast<int>(cfg_.heads), static_cast<int>(W / cfg_.heads),
+                   static_cast<int>(T))));
   grow(ctx_, W * T);
   grow(ff_, cfg_.intermediate * T);
   grow(sum_, W * T);
@@ -705,64 +705,12 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
     g.y = qkv_.get();
     g.positions = T;
     RunGemm(g, stream, prof, "enc_qkv");
-    {
-      // S^T[key][query] = sum_d K[d][key] Q[d][query], per head.
-      ConvParams p{};
-      p.x = qkv_.get();
-      p.w = qkv_.get() + static_cast<std::size_t>(W) * T;
-      p.y = scores_.get();
-      p.cin = hd;
-      p.len_in = T;
-      p.cout = T;
-      p.len_out = T;
-      p.ldw = T;
-      p.taps = 1;
-      p.phases = 1;
-      p.positions = T;
-      p.out_stride = 1;
-      p.batches = heads;
-      p.partial = partial_.get();
-      p.partial_capacity = kPartialFloats;
-      p.x_batch = static_cast<int64_t>(hd) * T;
-      p.w_batch = static_cast<int64_t>(hd) * T;
-      p.y_batch = static_cast<int64_t>(T) * T;
-      run("enc_scores", 2.0 * heads * hd * static_cast<double>(T) * T,
-          4.0 * (2.0 * W * T + static_cast<double>(heads) * T * T),
-          [&] { LaunchConv(p, stream); });
-    }
-    run("enc_softmax", 0.0, 8.0 * heads * static_cast<double>(T) * T, [&] {
-      LaunchColumnSoftmax(scores_.get(), heads, T, T,
-                          static_cast<float>(1.0 / std::sqrt(static_cast<double>(hd))), stream);
-    });
-    run("enc_transpose", 0.0, 8.0 * W * static_cast<double>(T), [&] {
-      LaunchTranspose(qkv_.get() + 2 * static_cast<std::size_t>(W) * T, W, T, T, vt_.get(),
-                      stream);
-    });
-    {
-      // O[d][query] = sum_key V[d][key] P[query][key], per head.
-      ConvParams p{};
-      p.x = scores_.get();
-      p.w = vt_.get();
-      p.y = ctx_.get();
-      p.cin = T;
-      p.len_in = T;
-      p.cout = hd;
-      p.len_out = T;
-      p.ldw = W;
-      p.taps = 1;
-      p.phases = 1;
-      p.positions = T;
-      p.out_stride = 1;
-      p.batches = heads;
-      p.partial = partial_.get();
-      p.partial_capacity = kPartialFloats;
-      p.x_batch = static_cast<int64_t>(T) * T;
-      p.w_batch = hd;
-      p.y_batch = static_cast<int64_t>(hd) * T;
-      run("enc_context", 2.0 * heads * hd * static_cast<double>(T) * T,
-          4.0 * (static_cast<double>(heads) * T * T + 2.0 * W * T),
-          [&] { LaunchConv(p, stream); });
-    }
+    HeadAttentionParams ap{qkv_.get(), qkv_.get() + static_cast<std::size_t>(W) * T,
+                           qkv_.get() + 2 * static_cast<std::size_t>(W) * T, ctx_.get(),
+                           heads_.get(), heads, hd, T,
+                           static_cast<float>(1.0 / std::sqrt(static_cast<double>(hd)))};
+    run("enc_attention", 4.0 * heads * hd * static_cast<double>(T) * T, 16.0 * W * T,
+        [&] { LaunchHeadAttention(ap, stream); });
     g = Gemm();
     g.d = &ly.out;
     g.x = ctx_.get();

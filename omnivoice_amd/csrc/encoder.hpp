@@ -51,14 +51,21 @@ struct ColumnNormParams {
 };
 void LaunchColumnNorm(const ColumnNormParams& p, hipStream_t stream);
 
-// Softmax over the rows of every column of `batches` [rows][cols]
-// matrices, of scale x, in place.
-void LaunchColumnSoftmax(float* x, int batches, int rows, int cols, float scale,
-                         hipStream_t stream);
-
-// y[c][r] = x[r][c] for r < rows, c < cols; x rows `ldx` apart.
-void LaunchTranspose(const float* x, int rows, int cols, int ldx, float* y,
-                     hipStream_t stream);
+// Softmax attention of `heads` heads over `steps` positions: out[d][t] =
+// sum_s v[d][s] softmax_s(scale sum_e k[e][s] q[e][t]), every operand
+// [heads][head_dim][steps]; `packed` is a workspace of
+// PackedHeadsElements(...) elements.
+struct HeadAttentionParams {
+  const float* q;
+  const float* k;
+  const float* v;
+  float* out;
+  std::uint16_t* packed;
+  int heads, head_dim, steps;
+  float scale;
+};
+std::size_t PackedHeadsElements(int heads, int head_dim, int steps);
+void LaunchHeadAttention(const HeadAttentionParams& p, hipStream_t stream);
 
 // y[c][f] = sum[c][f stride] scale for c < channels, f < frames; sum rows
 // `positions` long.

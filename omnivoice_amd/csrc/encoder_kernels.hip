@@ -2,15 +2,15 @@
 // gfx950 (the reference's kernels/encoder_kernels.hip counterparts: the
 // resampler that audio.cpp:265-322 runs on the host, GroupNorm + GELU,
 // LayerNorm, softmax, the frame pick and the RVQ nearest-entry search).
-// Every GEMM-shaped layer of the encoder runs on the fp32 matrix cores
-// through the convolution kernel; these kernels move each element once or
-// twice and are bound by HBM or, at the encoder's small sizes, by launch.
+// Every GEMM-shaped layer of the encoder but attention runs through the
+// convolution kernel; these kernels move each element once or twice and are
+// bound by HBM or, at the encoder's small sizes, by launch.
 //
-// The column kernels (LayerNorm over channels, softmax over keys) read a
-// channel-major matrix along its slow dimension: a work-group owns 8
-// adjacent columns, each column 32 lanes that hold every 32nd row in
-// registers, so each element is read once, all of a thread's loads are in
-// flight together, and the partial sums meet in LDS.
+// The column kernel (LayerNorm over channels) reads a channel-major matrix
+// along its slow dimension: a work-group owns 8 adjacent columns, each
+// column 32 lanes that hold every 32nd row in registers, so each element is
+// read once, all of a thread's loads are in flight together, and the partial
+// sums meet in LDS.
 #include <algorithm>
 #include <cfloat>
 #include <type_traits>
@@ -19,6 +19,7 @@
 #include "common.hpp"
 #include "encoder.hpp"
 #include "kernels.hpp"
+#include "split.hpp"
 
 namespace ovg {
 namespace {
@@ -106,7 +107,7 @@ __global__ __launch_bounds__(kThreads) void GroupNormGeluKernel(float* x, const 
     row[t] = Gelu(static_cast<float>((row[t] - mean) * inv * wc + bc));
 }
 
-// The column kernels: a work-group of kCols adjacent columns x kLanes lanes;
+// The column kernel: a work-group of kCols adjacent columns x kLanes lanes;
 // lane l of a column holds rows l, l + kLanes, ... (up to kPer of them) in
 // registers, so every element is read once with all its loads in flight.
 constexpr int kCols = 8;
@@ -177,93 +178,235 @@ __global__ __launch_bounds__(kThreads) void ColumnNormKernel(ColumnNormParams p)
   }
 }
 
-// Softmax down columns longer than the registers hold: three passes over
-// the rows, eight loads in flight per lane.
-__global__ __launch_bounds__(kThreads) void ColumnSoftmaxLongKernel(float* x, int rows, int cols,
-                                                                    float scale) {
-  __shared__ double scratch[kLanes][kCols];
-  __shared__ float peak[kLanes][kCols];
-  float* m = x + static_cast<size_t>(blockIdx.y) * rows * cols;
-  const int col = threadIdx.x % kCols, lane = threadIdx.x / kCols;
-  const int t = blockIdx.x * kCols + col;
-  const int tc = min(t, cols - 1);
-  float hi = -FLT_MAX;
-#pragma unroll 8
-  for (int r = lane; r < rows; r += kLanes)
-    hi = fmaxf(hi, m[static_cast<size_t>(r) * cols + tc]);
-  peak[lane][col] = hi;
-  __syncthreads();
-  for (int i = 0; i < kLanes; ++i)
-    hi = fmaxf(hi, peak[i][col]);
-  double s = 0.0;
-#pragma unroll 8
-  for (int r = lane; r < rows; r += kLanes)
-    s += expf((m[static_cast<size_t>(r) * cols + tc] - hi) * scale);
-  const float inv = static_cast<float>(1.0 / LaneSum(s, scratch));
-  if (t >= cols)
-    return;
-#pragma unroll 8
-  for (int r = lane; r < rows; r += kLanes) {
-    const size_t at = static_cast<size_t>(r) * cols + t;
-    m[at] = expf((m[at] - hi) * scale) * inv;
+// HuBERT's attention: the projections into matrix-core operands, then one
+// kernel over the heads, instead of scores, softmax, transpose and context
+// launches that move the [heads][steps][steps] scores through memory. Bound
+// by each wave's chain of dependent products and its softmax, hence eight
+// waves (two per SIMD) over the keys of only 32 queries. Both launches, 12
+// heads of 64 dims: 14.8, 20.7 and 47.1 us at 150, 500 and 1045 steps, against
+// 37.6, 52.9 and 156 us for the four launches (four waves: 15.8, 22.2, 59.2;
+// operands gathered and split by every work-group from the channel-major
+// projections: 24.9, 46.2, 119).
+//
+// Operand order, per head and tile of 32 positions (zeros past the head's
+// dims and past the last position), three parts (split.hpp) of 64 lanes x 16
+// bytes each:
+//   q, k  [16 dims s][part]: lane l is position l % 32, dims 16 s + 8 (l / 32)
+//         .. + 7
+//   v     [32 dims n][16 keys j][part]: lane l is dim 32 n + l % 32, keys 16 j
+//         + 8 (i / 4) + 4 (l / 32) + i % 4 for i < 8, the order in which the
+//         scores' accumulators hold the keys
+constexpr int kAttentionTile = 32;   // queries per work-group, keys per tile
+constexpr int kAttentionDims = 64;   // output dims per work-group
+constexpr int kAttentionThreads = 512;
+// 16-byte vectors of one tile of q or k and of v.
+__host__ __device__ constexpr int QkVectors(int head_dim) { return (head_dim + 15) / 16 * 192; }
+__host__ __device__ constexpr int ValueVectors(int head_dim) {
+  return (head_dim + 31) / 32 * 384;
+}
+
+__global__ __launch_bounds__(kThreads) void PackHeadsKernel(HeadAttentionParams p) {
+  const int T = p.steps, hd = p.head_dim;
+  const int tile = blockIdx.x, head = blockIdx.y, which = blockIdx.z;
+  const int tiles = gridDim.x;
+  const int t0 = tile * kAttentionTile;
+  const float* from = (which == 0 ? p.q : which == 1 ? p.k : p.v) +
+                      static_cast<size_t>(head) * hd * T;
+  uintx4* to = reinterpret_cast<uintx4*>(p.packed);
+  const size_t at = static_cast<size_t>(head) * tiles + tile;
+  const size_t heads_tiles = static_cast<size_t>(p.heads) * tiles;
+  if (which < 2)
+    to += (heads_tiles * which + at) * QkVectors(hd);
+  else
+    to += heads_tiles * 2 * QkVectors(hd) + at * ValueVectors(hd);
+  const int items = (which < 2 ? QkVectors(hd) : ValueVectors(hd)) / 3;
+  for (int e = threadIdx.x; e < items; e += kThreads) {
+    const int lane = e & 63, half = lane >> 5, l32 = lane & 31;
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      int d, t;
+      if (which < 2) {
+        d = (e >> 6) * 16 + 8 * half + i;
+        t = t0 + l32;
+      } else {
+        d = (e >> 7) * 32 + l32;
+        t = t0 + ((e >> 6) & 1) * 16 + 8 * (i >> 2) + 4 * half + (i & 3);
+      }
+      v[i] = from[static_cast<size_t>(min(d, hd - 1)) * T + min(t, T - 1)];
+      if (d >= hd || t >= T)
+        v[i] = 0.0F;
+    }
+    uintx4 part[3];
+    Split8(v, part);
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      to[((e >> 6) * 3 + k) * 64 + lane] = part[k];
   }
 }
 
-template <int kPer>
-__global__ __launch_bounds__(kThreads) void ColumnSoftmaxKernel(float* x, int rows, int cols,
-                                                                float scale) {
-  __shared__ double scratch[kLanes][kCols];
-  __shared__ float peak[kLanes][kCols];
-  float* m = x + static_cast<size_t>(blockIdx.y) * rows * cols;
-  const int col = threadIdx.x % kCols, lane = threadIdx.x / kCols;
-  const int t = blockIdx.x * kCols + col;
-  const int tc = min(t, cols - 1);
-  float v[kPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i)
-    v[i] = m[static_cast<size_t>(min(lane + i * kLanes, rows - 1)) * cols + tc];
-  float hi = -FLT_MAX;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i)
-    if (lane + i * kLanes < rows)
-      hi = fmaxf(hi, v[i]);
-  peak[lane][col] = hi;
-  __syncthreads();
-  for (int i = 0; i < kLanes; ++i)
-    hi = fmaxf(hi, peak[i][col]);
-  double s = 0.0;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    v[i] = expf((v[i] - hi) * scale);
-    if (lane + i * kLanes < rows)
-      s += v[i];
+// A work-group owns one head's 32 queries (and 64 of the head's dims; wider
+// heads take more work-groups); its eight waves take every eighth tile of
+// 32 keys. Scores are formed transposed (S^T = K^T Q, each lane one query
+// column) and never leave registers: they become the operand of O = V P^T
+// there. The softmax runs online per wave (a running maximum, the sum in
+// double, the output rescaled when the maximum grows), and the waves'
+// states meet in LDS at the end. The queries are in LDS (kQueriesInLds: up to
+// 256 dims), a tile's keys and values come straight into registers, the next
+// keys during the softmax.
+template <bool kQueriesInLds>
+__global__ __launch_bounds__(kAttentionThreads) void HeadAttentionKernel(HeadAttentionParams p) {
+  constexpr int kWaves = kAttentionThreads / 64;
+  // The queries, then (once every wave is past them) the waves' outputs.
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ float peaks[kWaves][kAttentionTile];
+  __shared__ double sums[kWaves][kAttentionTile];
+  auto merged = reinterpret_cast<float(*)[kAttentionDims][kAttentionTile]>(lds);
+  const int T = p.steps, hd = p.head_dim;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5, l32 = lane & 31;
+  const int tiles = gridDim.x, head = blockIdx.y;
+  const int q0 = blockIdx.x * kAttentionTile;
+  const int slab = blockIdx.z * kAttentionDims;  // first output dim
+  const int rounds = (hd + 15) / 16;             // 16 dims each
+  const int blocks = (hd + 31) / 32;             // 32 output dims each
+  const size_t heads_tiles = static_cast<size_t>(p.heads) * tiles;
+  const uintx4* packed = reinterpret_cast<const uintx4*>(p.packed);
+  const size_t first = static_cast<size_t>(head) * tiles;
+  const uintx4* queries = packed + (first + blockIdx.x) * QkVectors(hd);
+  const uintx4* keys = packed + (heads_tiles + first) * QkVectors(hd) + lane;
+  const uintx4* values = packed + heads_tiles * 2 * QkVectors(hd) + first * ValueVectors(hd) + lane;
+  uintx4* const staged = reinterpret_cast<uintx4*>(lds);
+  if constexpr (kQueriesInLds) {
+    for (int e = threadIdx.x; e < rounds * 192; e += kAttentionThreads)
+      staged[e] = queries[e];
+    __syncthreads();
   }
-  const float inv = static_cast<float>(1.0 / LaneSum(s, scratch));
-  if (t >= cols)
-    return;
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int r = lane + i * kLanes;
-    if (r < rows)
-      m[static_cast<size_t>(r) * cols + t] = v[i] * inv;
-  }
-}
+  const int n_last = blocks - 1;
 
-__global__ __launch_bounds__(kThreads) void TransposeKernel(const float* x, int rows, int cols,
-                                                            int ldx, float* y) {
-  __shared__ float tile[32][33];
-  const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
-  const int tx = threadIdx.x % 32, ty = threadIdx.x / 32;  // 8 rows per pass
-  for (int i = ty; i < 32; i += 8) {
-    const int r = r0 + i, c = c0 + tx;
-    if (r < rows && c < cols)
-      tile[i][tx] = x[static_cast<size_t>(r) * ldx + c];
+  uintx4 kf[4][3];
+  auto load_keys = [&](int tile, int s0) {
+    const uintx4* from = keys + static_cast<size_t>(min(tile, tiles - 1)) * QkVectors(hd);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        kf[s][k] = from[(min(s0 + s, rounds - 1) * 3 + k) * 64];
+  };
+  floatx16 main[2] = {}, corr[2] = {};
+  float peak = -FLT_MAX;
+  double sum = 0.0;
+  load_keys(wave, 0);
+  for (int tile = wave; tile < tiles; tile += kWaves) {
+    const int k0 = tile * kAttentionTile;
+    // Values of this tile, in flight during the scores and the softmax.
+    uintx4 vf[2][2][3];
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const uintx4* from = values + static_cast<size_t>(tile) * ValueVectors(hd) +
+                           min(slab / 32 + n, n_last) * 384;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          vf[n][j][k] = from[(j * 3 + k) * 64];
+    }
+    floatx16 sm = {}, sc = {};
+    for (int s0 = 0; s0 < rounds; s0 += 4) {
+#pragma unroll
+      for (int s = 0; s < 4; ++s) {
+        if (s0 + s >= rounds)
+          break;
+        uintx4 qf[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+          qf[k] = kQueriesInLds ? staged[((s0 + s) * 3 + k) * 64 + lane]
+                                : queries[((s0 + s) * 3 + k) * 64 + lane];
+        sc = MfmaBf16(kf[s][2], qf[0], sc);
+        sm = MfmaBf16(kf[s][0], qf[0], sm);
+        sc = MfmaBf16(kf[s][0], qf[2], sc);
+        sc = MfmaBf16(kf[s][1], qf[1], sc);
+        sc = MfmaBf16(kf[s][1], qf[0], sc);
+        sc = MfmaBf16(kf[s][0], qf[1], sc);
+      }
+      // The next round of dims, or the next tile's first one.
+      if (s0 + 4 < rounds)
+        load_keys(tile, s0 + 4);
+      else
+        load_keys(tile + kWaves, 0);
+    }
+    float s[16], top = peak;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = Join(sm[r], sc[r]);
+      if (k0 + 8 * (r >> 2) + 4 * half + (r & 3) < T)
+        top = fmaxf(top, s[r]);
+    }
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float keep = expf((peak - top) * p.scale);
+    peak = top;
+    double part = 0.0;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < T ? expf((s[r] - top) * p.scale) : 0.0F;
+      part += s[r];
+    }
+    sum = sum * keep + (part + __shfl_xor(part, 32));
+#pragma unroll
+    for (int n = 0; n < 2; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        main[n][r] *= keep;
+        corr[n][r] *= keep;
+      }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      uintx4 pf[3];
+      Split8(s + 8 * j, pf);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        corr[n] = MfmaBf16(vf[n][j][2], pf[0], corr[n]);
+        main[n] = MfmaBf16(vf[n][j][0], pf[0], main[n]);
+        corr[n] = MfmaBf16(vf[n][j][0], pf[2], corr[n]);
+        corr[n] = MfmaBf16(vf[n][j][1], pf[1], corr[n]);
+        corr[n] = MfmaBf16(vf[n][j][1], pf[0], corr[n]);
+        corr[n] = MfmaBf16(vf[n][j][0], pf[1], corr[n]);
+      }
+    }
   }
   __syncthreads();
-  for (int i = ty; i < 32; i += 8) {
-    const int c = c0 + i, r = r0 + tx;
-    if (r < rows && c < cols)
-      y[static_cast<size_t>(c) * rows + r] = tile[tx][i];
+#pragma unroll
+  for (int n = 0; n < 2; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r)
+      merged[wave][32 * n + 8 * (r >> 2) + 4 * half + (r & 3)][l32] = Join(main[n][r], corr[n][r]);
+  if (half == 0) {
+    peaks[wave][l32] = peak;
+    sums[wave][l32] = sum;
+  }
+  __syncthreads();
+  const int q = threadIdx.x % kAttentionTile;
+  float top = peaks[0][q];
+#pragma unroll
+  for (int w = 1; w < kWaves; ++w)
+    top = fmaxf(top, peaks[w][q]);
+  float keep[kWaves];
+  double total = 0.0;
+#pragma unroll
+  for (int w = 0; w < kWaves; ++w) {
+    keep[w] = expf((peaks[w][q] - top) * p.scale);
+    total += sums[w][q] * keep[w];
+  }
+  const float inv = static_cast<float>(1.0 / total);
+  for (int d = threadIdx.x / kAttentionTile; d < kAttentionDims;
+       d += kAttentionThreads / kAttentionTile) {
+    float o = 0.0F;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+      o += merged[w][d][q] * keep[w];
+    if (q0 + q < T && slab + d < hd)
+      p.out[(static_cast<size_t>(head) * hd + slab + d) * T + q0 + q] = o * inv;
   }
 }
 
@@ -330,9 +473,7 @@ __global__ __launch_bounds__(kThreads) void NearestKernel(NearestParams p) {
     p.residual[static_cast<size_t>(h) * p.frames + f] -= row[h];
 }
 
-// Register-cached column kernels hold up to 64 rows per lane: 2048 rows
-// (LayerNorm, which also holds its weights and running sums: 1024).
-constexpr int kMaxColumnRows = 64 * kLanes;
+// The column kernel holds up to 32 rows per lane: 1024 channels.
 constexpr int kMaxNormChannels = 32 * kLanes;
 
 template <typename K>
@@ -341,10 +482,8 @@ void ColumnDispatch(int rows, K&& launch) {
     launch(std::integral_constant<int, 8>());
   else if (rows <= 16 * kLanes)
     launch(std::integral_constant<int, 16>());
-  else if (rows <= 32 * kLanes)
-    launch(std::integral_constant<int, 32>());
   else
-    launch(std::integral_constant<int, 64>());
+    launch(std::integral_constant<int, 32>());
 }
 
 int Blocks(size_t work) {
@@ -386,35 +525,33 @@ void LaunchColumnNorm(const ColumnNormParams& p, hipStream_t stream) {
   Require(p.channels >= 1 && p.channels <= kMaxNormChannels && p.positions >= 1,
           "layer norm: 1 to 1024 channels");
   ColumnDispatch(p.channels, [&](auto per) {
-    if constexpr (decltype(per)::value <= kMaxNormChannels / kLanes)
-      Dispatch(ColumnNormKernel<decltype(per)::value>, dim3((p.positions + kCols - 1) / kCols),
-               dim3(kThreads), 0, stream, true, true, p);
+    Dispatch(ColumnNormKernel<decltype(per)::value>, dim3((p.positions + kCols - 1) / kCols),
+             dim3(kThreads), 0, stream, true, true, p);
   });
 }
 
-void LaunchColumnSoftmax(float* x, int batches, int rows, int cols, float scale,
-                         hipStream_t stream) {
-  Require(x != nullptr, "softmax: null pointer");
-  Require(batches >= 1 && batches <= 65535 && rows >= 1 && cols >= 1, "softmax: bad shape");
-  if (rows > kMaxColumnRows) {
-    Dispatch(ColumnSoftmaxLongKernel, dim3((cols + kCols - 1) / kCols, batches), dim3(kThreads),
-             0, stream, true, true, x, rows, cols, scale);
-    return;
-  }
-  ColumnDispatch(rows, [&](auto per) {
-    Dispatch(ColumnSoftmaxKernel<decltype(per)::value>,
-             dim3((cols + kCols - 1) / kCols, batches), dim3(kThreads), 0, stream, true, true, x,
-             rows, cols, scale);
-  });
+std::size_t PackedHeadsElements(int heads, int head_dim, int steps) {
+  const std::size_t tiles = (static_cast<std::size_t>(steps) + kAttentionTile - 1) / kAttentionTile;
+  return heads * tiles * (2 * QkVectors(head_dim) + ValueVectors(head_dim)) * 8;
 }
 
-void LaunchTranspose(const float* x, int rows, int cols, int ldx, float* y,
-                     hipStream_t stream) {
-  Require(x && y, "transpose: null pointer");
-  Require(rows >= 1 && cols >= 1 && ldx >= cols && (rows + 31) / 32 <= 65535,
-          "transpose: bad shape");
-  Dispatch(TransposeKernel, dim3((cols + 31) / 32, (rows + 31) / 32), dim3(kThreads), 0, stream,
-           true, true, x, rows, cols, ldx, y);
+void LaunchHeadAttention(const HeadAttentionParams& p, hipStream_t stream) {
+  Require(p.q && p.k && p.v && p.packed && p.out, "attention: null pointer");
+  const int slabs = (p.head_dim + kAttentionDims - 1) / kAttentionDims;
+  Require(p.heads >= 1 && p.heads <= 65535 && p.head_dim >= 1 && slabs <= 65535 &&
+              p.steps >= 1,
+          "attention: bad shape");
+  const unsigned tiles = (p.steps + kAttentionTile - 1) / kAttentionTile;
+  Dispatch(PackHeadsKernel, dim3(tiles, p.heads, 3), dim3(kThreads), 0, stream, true, false, p);
+  const dim3 grid(tiles, p.heads, slabs);
+  const std::uint32_t merge = kAttentionThreads / 64 * kAttentionDims * kAttentionTile * 4;
+  const std::uint32_t queries = QkVectors(p.head_dim) * 16;
+  if (p.head_dim <= 256)
+    Dispatch(HeadAttentionKernel<true>, grid, dim3(kAttentionThreads), std::max(merge, queries),
+             stream, false, true, p);
+  else
+    Dispatch(HeadAttentionKernel<false>, grid, dim3(kAttentionThreads), merge, stream, false,
+             true, p);
 }
 
 void LaunchPickFrames(const double* sum, int channels, int positions, int stride, int frames,

@@ -61,6 +61,21 @@ def test_tiny_encode_matches_oracle(frames):
     compare(got, want)
 
 
+@pytest.mark.parametrize("width,heads,frames", [
+    (16, 4, 15),   # 30 steps: less than one key tile; heads of 4 dims
+    (16, 4, 16),   # 32 steps: one whole tile
+    (64, 1, 66),   # 64 dims, a wave with two tiles, the last one ragged
+    (96, 1, 33),   # heads wider than one round of dims, two output slabs
+    (160, 2, 130), # 80 dims, more than two rounds of the waves
+    (320, 1, 40),  # queries not in LDS
+])
+def test_attention_shapes_match_oracle(width, heads, frames):
+    cfg = dict(oracle.encoder_tiny_config(), width=width, heads=heads)
+    x = signal(frames * cfg["frame_samples"], frames)
+    got = ov.Encoder.synthetic(cfg, 21).encode(x, intermediates=True)
+    compare(got, oracle.Encoder(cfg, 21).encode(x))
+
+
 def test_encode_matches_transformers_fixture():
     """The GPU encoder against transformers' HubertModel and DacEncoder plus
     torch float64 layers on the same synthetic weights

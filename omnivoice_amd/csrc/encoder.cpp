@@ -17,7 +17,7 @@
 //    convolution, residual additions by its accumulation.
 // The mean of HuBERT's states is summed in double by the LayerNorm that
 // produces each state. The nearest-entry search compares distances in
-// double.
+// double, all its stages in one kernel.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -111,9 +111,9 @@ struct Block {
   int channels = 0, stride = 1;
 };
 struct Stage {
-  Dense project;
-  DeviceBuffer<float> embed, table;  // [entries][dim], [entries][hidden]
-  DeviceBuffer<double> norms;        // [entries]
+  DeviceBuffer<float> project, bias;  // [hidden][dim], [dim]
+  DeviceBuffer<float> embed, table;   // [dim][entries], [entries][hidden]
+  DeviceBuffer<double> norms;         // [entries]
 };
 
 // Shapes of one encode of `length` samples.
@@ -183,14 +183,15 @@ class EncoderEngine {
   DeviceBuffer<float> ac_alpha_;
   Dense ac_out_, fc_;
   std::vector<std::unique_ptr<Stage>> stages_;
+  DeviceBuffer<RvqStage> stage_list_;
   // work buffers
   DeviceBuffer<float> samples_, wave_, fa_, fb_, cols_, tmp_, h_, qkv_, ctx_, ff_;
   DeviceBuffer<double> sum_;
   DeviceBuffer<std::uint16_t> heads_;  // the attention's operands
   // Split-K workspace of the thin GEMMs (HuBERT at short lengths, the
-  // semantic encoder, the quantizer's projections).
+  // semantic encoder).
   DeviceBuffer<float> partial_;
-  DeviceBuffer<float> sem_, st_, t1_, x_, xa_, ya_, joint_, emb_, resid_, proj_;
+  DeviceBuffer<float> sem_, st_, t1_, x_, xa_, ya_, joint_, emb_, resid_;
   DeviceBuffer<std::int32_t> codes_;
 };
 
@@ -431,14 +432,19 @@ EncoderEngine::EncoderEngine(const ovc_encoder_config& cfg, std::uint64_t seed,
     });
   for (auto& w : workers)
     w.join();
+  std::vector<RvqStage> stage_list;
   for (int q = 0; q < cfg.codebooks; ++q) {
     auto st = std::make_unique<Stage>();
-    MakeDense(pw[q], &pb[q], D, H, 1, &st->project);
-    Upload(st->embed, emb[q]);
+    Upload(st->project, ConvLayout(pw[q], D, H, 1));
+    Upload(st->bias, pb[q]);
+    Upload(st->embed, ConvLayout(emb[q], E, D, 1));
     Upload(st->table, tables[q]);
     Upload(st->norms, norms[q]);
+    stage_list.push_back({st->project.get(), st->bias.get(), st->embed.get(), st->norms.get(),
+                          st->table.get()});
     stages_[q] = std::move(st);
   }
+  Upload(stage_list_, stage_list);
   partial_.Reserve(kPartialFloats);
   Check(hipDeviceSynchronize(), "encoder upload");
 }
@@ -524,7 +530,6 @@ void EncoderEngine::Reserve(const Plan& p) {
   grow(joint_, H_ * F);
   grow(emb_, H_ * F);
   grow(resid_, H_ * F);
-  grow(proj_, cfg_.codebook_dim * F);
   grow(codes_, cfg_.codebooks * F);
 }
 
@@ -840,24 +845,12 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
     g.positions = F;
     RunGemm(g, stream, prof, "enc_fc");
   }
-  // (a copy, not a kernel: the profiler times kernels only)
-  Check(hipMemcpyAsync(resid_.get(), emb_.get(), sizeof(float) * H * F, hipMemcpyDeviceToDevice,
-                       stream),
-        "copy embeddings");
   const int D = static_cast<int>(cfg_.codebook_dim), E = static_cast<int>(cfg_.codebook_size);
-  for (std::size_t q = 0; q < stages_.size(); ++q) {
-    const Stage& st = *stages_[q];
-    Gemm g;
-    g.d = &st.project;
-    g.x = resid_.get();
-    g.y = proj_.get();
-    g.positions = F;
-    RunGemm(g, stream, prof, "enc_rvq_project");
-    NearestParams np{proj_.get(), st.embed.get(), st.norms.get(), st.table.get(), resid_.get(),
-                     codes + q * F, D, E, H, F};
-    run("enc_rvq_nearest", 2.0 * D * static_cast<double>(E) * F,
-        4.0 * (static_cast<double>(E) * D * F + 2.0 * H * F), [&] { LaunchNearest(np, stream); });
-  }
+  const int Q = static_cast<int>(stages_.size());
+  RvqEncodeParams qp{emb_.get(), stage_list_.get(), resid_.get(), codes, Q, D, E, H, F};
+  run("enc_rvq", 2.0 * Q * D * static_cast<double>(H + E) * F,
+      4.0 * (static_cast<double>(Q) * D * (H + E) + static_cast<double>(H + Q) * F),
+      [&] { LaunchRvqEncode(qp, stream); });
 }
 
 void EncoderEngine::Encode(const float* samples, int64_t length, std::int32_t* codes,

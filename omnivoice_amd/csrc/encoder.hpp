@@ -72,20 +72,26 @@ void LaunchHeadAttention(const HeadAttentionParams& p, hipStream_t stream);
 void LaunchPickFrames(const double* sum, int channels, int positions, int stride, int frames,
                       double scale, float* y, hipStream_t stream);
 
-// One residual vector quantizer stage: for every frame f the entry e of the
-// largest -((|p|^2 - 2 p.e) + |e|^2) (the nearest; the lowest index on
-// ties, distances in double) of the projected residual p = proj[:, f];
-// codes[f] = e and residual[:, f] -= table[e].
-struct NearestParams {
-  const float* proj;       // [dim][frames]
-  const float* embed;      // [entries][dim]
-  const double* norms;     // [entries], |e|^2
-  const float* table;      // [entries][hidden]
-  float* residual;         // [hidden][frames]
-  std::int32_t* codes;     // [frames]
-  int dim, entries, hidden, frames;
+// The residual vector quantizer: for every frame f and stage in turn, the
+// projected residual v = bias + project^T r, the entry e of the largest
+// -((|v|^2 - 2 v.e) + |e|^2) (the nearest; the lowest index on ties,
+// distances in double), codes[stage][f] = e and r -= table[e]; r starts as
+// x[:, f].
+struct RvqStage {
+  const float* project;  // [hidden][dim]
+  const float* bias;     // [dim]
+  const float* embed;    // [dim][entries]
+  const double* norms;   // [entries], |e|^2
+  const float* table;    // [entries][hidden]
 };
-void LaunchNearest(const NearestParams& p, hipStream_t stream);
+struct RvqEncodeParams {
+  const float* x;         // [hidden][frames]
+  const RvqStage* stage;  // [stages], device memory
+  float* residual;        // [frames][hidden], workspace
+  std::int32_t* codes;    // [stages][frames]
+  int stages, dim, entries, hidden, frames;
+};
+void LaunchRvqEncode(const RvqEncodeParams& p, hipStream_t stream);
 
 }  // namespace ovg
 

@@ -1,7 +1,7 @@
 // The audio encoder's element-wise, normalisation and selection kernels on
 // gfx950 (the reference's kernels/encoder_kernels.hip counterparts: the
 // resampler that audio.cpp:265-322 runs on the host, GroupNorm + GELU,
-// LayerNorm, softmax, the frame pick and the RVQ nearest-entry search).
+// LayerNorm, attention, the frame pick and the residual vector quantizer).
 // Every GEMM-shaped layer of the encoder but attention runs through the
 // convolution kernel; these kernels move each element once or twice and are
 // bound by HBM or, at the encoder's small sizes, by launch.
@@ -422,55 +422,156 @@ __global__ __launch_bounds__(kThreads) void PickFramesKernel(const double* sum, 
   }
 }
 
-constexpr int kMaxDim = 1024;
+// The residual vector quantizer, every stage of FRAMES frames in one
+// work-group: a frame's stages depend on each other, frames do not. Per stage
+// the projection (float32 sums over an eighth of the input per wave, the
+// eight added in order), the distances to every entry (double, dims in
+// order), the nearest entry (the lowest index on ties) and the subtraction of
+// its decoded row from the residual, which stays in LDS (in `residual` where
+// it does not fit, kInLds false).
+//
+// A stage reads the projection and the codebook once per work-group (512 KB
+// at 1024 x 64 x 1024, 4 us of the CU's 64 B/clk load path) in a chain of
+// load batches, barriers and the search's reduction, whose latency bounds the
+// kernel at about 14 us per stage. All eight stages: 113 us at 75 and 250
+// frames against 262 and 277 us for a projection and a search launch each;
+// 163 us at 523 frames (400 us), where more frames than CUs go two to a
+// work-group. Batches of 64 and 32 loads (350 us: the unrolled code no longer
+// fits the instruction cache) and 16-byte loads (122 us, 291 us at 523
+// frames) were slower.
+constexpr int kRvqThreads = 512;
+constexpr int kRvqWaves = kRvqThreads / 64;
+constexpr int kRvqMaxDim = 1024;
+constexpr std::uint32_t kRvqLdsLimit = 144 * 1024;
+constexpr std::uint64_t RvqLdsBytes(int frames, int dim, std::int64_t hidden) {
+  return static_cast<std::uint64_t>(frames) *
+         (dim * (8 + 4 * kRvqWaves) + 4 * static_cast<std::uint64_t>(hidden));
+}
 
-__global__ __launch_bounds__(kThreads) void NearestKernel(NearestParams p) {
-  __shared__ double v[kMaxDim];
-  __shared__ double scratch[kThreads / 64];
-  __shared__ double best_d[kThreads];
-  __shared__ int best_e[kThreads];
-  const int f = blockIdx.x;
-  double pp = 0.0;
-  for (int d = threadIdx.x; d < p.dim; d += kThreads) {
-    const double x = p.proj[static_cast<size_t>(d) * p.frames + f];
-    v[d] = x;
-    pp += x * x;
-  }
-  // |p|^2 summed in a fixed order: lane partials, then the waves in turn.
-  pp = BlockSum(pp, scratch);
-  double best = -DBL_MAX;
-  int arg = 0;
-  for (int e = threadIdx.x; e < p.entries; e += kThreads) {
-    const float* row = p.embed + static_cast<size_t>(e) * p.dim;
-    double dot = 0.0;
-    for (int d = 0; d < p.dim; ++d)
-      dot += v[d] * row[d];
-    const double dist = -((pp - 2.0 * dot) + p.norms[e]);
-    if (dist > best) {  // entries ascend per thread: ties keep the lower
-      best = dist;
-      arg = e;
+template <int FRAMES, bool kInLds>
+__global__ __launch_bounds__(kRvqThreads) void RvqEncodeKernel(RvqEncodeParams p) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ double best_d[FRAMES][kRvqWaves];
+  __shared__ int best_e[FRAMES][kRvqWaves];
+  const int D = p.dim, E = p.entries, H = p.hidden;
+  double* const v = reinterpret_cast<double*>(lds);                  // [FRAMES][D]
+  float* const part = reinterpret_cast<float*>(v + FRAMES * D);      // [waves][FRAMES][D]
+  float* const lds_r = part + kRvqWaves * FRAMES * D;                // [FRAMES][H]
+  const int f0 = blockIdx.x * FRAMES;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  auto residual = [&](int f, int h) -> float& {
+    if constexpr (kInLds)
+      return lds_r[f * H + h];
+    else
+      return p.residual[static_cast<size_t>(min(f0 + f, p.frames - 1)) * H + h];
+  };
+#pragma unroll
+  for (int f = 0; f < FRAMES; ++f)
+    for (int h = tid; h < H; h += kRvqThreads)
+      residual(f, h) = p.x[static_cast<size_t>(h) * p.frames + min(f0 + f, p.frames - 1)];
+  const int per = (H + kRvqWaves - 1) / kRvqWaves;
+  const int h_begin = min(wave * per, H), h_end = min(h_begin + per, H);
+  for (int q = 0; q < p.stages; ++q) {
+    const RvqStage st = p.stage[q];
+    __syncthreads();
+    for (int d0 = 0; d0 < D; d0 += 64) {
+      const int d = min(d0 + lane, D - 1);
+      float acc[FRAMES] = {};
+#pragma unroll 16
+      for (int h = h_begin; h < h_end; ++h) {
+        const float w = st.project[static_cast<size_t>(h) * D + d];
+#pragma unroll
+        for (int f = 0; f < FRAMES; ++f)
+          acc[f] = fmaf(w, residual(f, h), acc[f]);
+      }
+      if (d0 + lane < D)
+#pragma unroll
+        for (int f = 0; f < FRAMES; ++f)
+          part[(wave * FRAMES + f) * D + d] = acc[f];
     }
-  }
-  best_d[threadIdx.x] = best;
-  best_e[threadIdx.x] = arg;
-  __syncthreads();
-  for (int half = kThreads / 2; half > 0; half >>= 1) {
-    if (threadIdx.x < half) {
-      const double od = best_d[threadIdx.x + half];
-      const int oe = best_e[threadIdx.x + half];
-      if (od > best_d[threadIdx.x] || (od == best_d[threadIdx.x] && oe < best_e[threadIdx.x])) {
-        best_d[threadIdx.x] = od;
-        best_e[threadIdx.x] = oe;
+    __syncthreads();
+    for (int i = tid; i < FRAMES * D; i += kRvqThreads) {
+      float sum = 0.0F;
+#pragma unroll
+      for (int w = 0; w < kRvqWaves; ++w)
+        sum += part[w * FRAMES * D + i];
+      v[i] = sum + st.bias[i % D];
+    }
+    __syncthreads();
+    double best[FRAMES];
+    int arg[FRAMES];
+#pragma unroll
+    for (int f = 0; f < FRAMES; ++f) {
+      best[f] = -DBL_MAX;
+      arg[f] = 0;
+    }
+    // Entries tid and tid + 512 of every 1024, their loads interleaved.
+    for (int e0 = tid; e0 < E; e0 += 2 * kRvqThreads) {
+      const int e1 = e0 + kRvqThreads;
+      const float* c0 = st.embed + e0;
+      const float* c1 = st.embed + min(e1, E - 1);
+      double pp[FRAMES] = {}, dot0[FRAMES] = {}, dot1[FRAMES] = {};
+#pragma unroll 8
+      for (int d = 0; d < D; ++d) {
+        const double w0 = c0[static_cast<size_t>(d) * E], w1 = c1[static_cast<size_t>(d) * E];
+#pragma unroll
+        for (int f = 0; f < FRAMES; ++f) {
+          const double x = v[f * D + d];
+          pp[f] += x * x;
+          dot0[f] += x * w0;
+          dot1[f] += x * w1;
+        }
+      }
+      // Entries ascend per thread: ties keep the lower.
+#pragma unroll
+      for (int f = 0; f < FRAMES; ++f) {
+        const double dist0 = -((pp[f] - 2.0 * dot0[f]) + st.norms[e0]);
+        if (dist0 > best[f]) {
+          best[f] = dist0;
+          arg[f] = e0;
+        }
+        const double dist1 = -((pp[f] - 2.0 * dot1[f]) + st.norms[min(e1, E - 1)]);
+        if (e1 < E && dist1 > best[f]) {
+          best[f] = dist1;
+          arg[f] = e1;
+        }
+      }
+    }
+#pragma unroll
+    for (int f = 0; f < FRAMES; ++f) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        const double od = __shfl_xor(best[f], o);
+        const int oe = __shfl_xor(arg[f], o);
+        if (od > best[f] || (od == best[f] && oe < arg[f])) {
+          best[f] = od;
+          arg[f] = oe;
+        }
+      }
+      if (lane == 0) {
+        best_d[f][wave] = best[f];
+        best_e[f][wave] = arg[f];
       }
     }
     __syncthreads();
+#pragma unroll
+    for (int f = 0; f < FRAMES; ++f) {
+      double top = best_d[f][0];
+      int code = best_e[f][0];
+#pragma unroll
+      for (int w = 1; w < kRvqWaves; ++w)
+        if (best_d[f][w] > top || (best_d[f][w] == top && best_e[f][w] < code)) {
+          top = best_d[f][w];
+          code = best_e[f][w];
+        }
+      if (tid == 0 && f0 + f < p.frames)
+        p.codes[static_cast<size_t>(q) * p.frames + f0 + f] = code;
+      if (kInLds || f0 + f < p.frames)
+        for (int h = tid; h < H; h += kRvqThreads)
+          residual(f, h) -= st.table[static_cast<size_t>(code) * H + h];
+    }
   }
-  const int code = best_e[0];
-  if (threadIdx.x == 0)
-    p.codes[f] = code;
-  const float* row = p.table + static_cast<size_t>(code) * p.hidden;
-  for (int h = threadIdx.x; h < p.hidden; h += kThreads)
-    p.residual[static_cast<size_t>(h) * p.frames + f] -= row[h];
 }
 
 // The column kernel holds up to 32 rows per lane: 1024 channels.
@@ -565,12 +666,23 @@ void LaunchPickFrames(const double* sum, int channels, int positions, int stride
            scale, y);
 }
 
-void LaunchNearest(const NearestParams& p, hipStream_t stream) {
-  Require(p.proj && p.embed && p.norms && p.table && p.residual && p.codes,
-          "nearest: null pointer");
-  Require(p.dim >= 1 && p.dim <= kMaxDim && p.entries >= 1 && p.hidden >= 1 && p.frames >= 1,
-          "nearest: bad shape");
-  Dispatch(NearestKernel, dim3(p.frames), dim3(kThreads), 0, stream, true, true, p);
+void LaunchRvqEncode(const RvqEncodeParams& p, hipStream_t stream) {
+  Require(p.x && p.stage && p.residual && p.codes, "quantizer: null pointer");
+  Require(p.dim >= 1 && p.dim <= kRvqMaxDim && p.entries >= 1 && p.hidden >= 1 &&
+              p.frames >= 1 && p.stages >= 1,
+          "quantizer: bad shape");
+  auto launch = [&](auto kernel, int frames, std::uint64_t bytes) {
+    Dispatch(kernel, dim3((p.frames + frames - 1) / frames), dim3(kRvqThreads),
+             static_cast<std::uint32_t>(bytes), stream, true, true, p);
+  };
+  // Two frames per work-group once one each would take more than one round of
+  // the CUs.
+  if (p.frames > kCus && RvqLdsBytes(2, p.dim, p.hidden) <= kRvqLdsLimit)
+    launch(RvqEncodeKernel<2, true>, 2, RvqLdsBytes(2, p.dim, p.hidden));
+  else if (RvqLdsBytes(1, p.dim, p.hidden) <= kRvqLdsLimit)
+    launch(RvqEncodeKernel<1, true>, 1, RvqLdsBytes(1, p.dim, p.hidden));
+  else
+    launch(RvqEncodeKernel<1, false>, 1, RvqLdsBytes(1, p.dim, 0));
 }
 
 }  // namespace ovg

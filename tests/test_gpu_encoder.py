@@ -76,6 +76,18 @@ def test_attention_shapes_match_oracle(width, heads, frames):
     compare(got, oracle.Encoder(cfg, 21).encode(x))
 
 
+@pytest.mark.parametrize("frames,dim,size", [
+    (9, 70, 1500),   # dims and entries past one round of the lanes and threads
+    (300, 8, 1024),  # two frames per work-group
+    (257, 65, 513),  # the last work-group holds one frame
+])
+def test_quantizer_shapes_match_oracle(frames, dim, size):
+    cfg = dict(oracle.encoder_tiny_config(), codebook_dim=dim, codebook_size=size)
+    x = signal(frames * cfg["frame_samples"], frames)
+    got = ov.Encoder.synthetic(cfg, 22).encode(x, intermediates=True)
+    compare(got, oracle.Encoder(cfg, 22).encode(x))
+
+
 def test_encode_matches_transformers_fixture():
     """The GPU encoder against transformers' HubertModel and DacEncoder plus
     torch float64 layers on the same synthetic weights

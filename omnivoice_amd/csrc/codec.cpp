@@ -61,7 +61,7 @@ constexpr int kDilations[3] = {1, 3, 9};
 // with ka = (p + pad) % s and c = (p + pad) / s. Tap 0 is the one at offset
 // c - 1. Weights [in][out][2s] -> [phase][tap][in][out].
 struct UpsampleTaps {
-  int offsets[kConvMaxPhases][2];
+  int first[kConvMaxPhases];
   int kernel_index[kConvMaxPhases][2];
 };
 UpsampleTaps Phases(int stride) {
@@ -70,9 +70,8 @@ UpsampleTaps Phases(int stride) {
   for (int p = 0; p < stride; ++p) {
     const int ka = (p + pad) % stride;
     const int c = (p + pad) / stride;
-    u.offsets[p][0] = c - 1;
+    u.first[p] = c - 1;
     u.kernel_index[p][0] = ka + stride;
-    u.offsets[p][1] = c;
     u.kernel_index[p][1] = ka;
   }
   return u;
@@ -90,7 +89,8 @@ std::vector<float> UpsampleLayout(const std::vector<float>& w, int in, int out, 
 }
 
 struct Conv {
-  DeviceBuffer<float> w, b;  // [taps][in][out], [out]
+  DeviceBuffer<ConvUnit> w;
+  DeviceBuffer<float> b;  // [out]
   int in = 0, out = 0, taps = 1, dilation = 1;
 };
 struct Unit {
@@ -98,7 +98,8 @@ struct Unit {
   Conv conv1, conv2;
 };
 struct Block {
-  DeviceBuffer<float> alpha, w, b;  // w [stride][2][in][out]
+  DeviceBuffer<ConvUnit> w;  // a lead per phase, two taps
+  DeviceBuffer<float> alpha, b;
   int in = 0, out = 0, stride = 1;
   Unit units[3];
 };
@@ -108,7 +109,7 @@ void LoadConv(const Source& src, const std::string& prefix, std::uint64_t id, in
   const auto w = src.Get(prefix + ".weight", {out, in, kernel}, id,
                          gain / std::sqrt(static_cast<double>(in) * kernel));
   const auto b = src.Get(prefix + ".bias", {out}, id + 1, 0.01);
-  Upload(conv->w, ConvLayout(w, out, in, kernel));
+  UploadConv(conv->w, ConvLayout(w, out, in, kernel), 1, kernel, in, out);
   Upload(conv->b, b);
   conv->in = in;
   conv->out = out;
@@ -221,7 +222,7 @@ CodecEngine::CodecEngine(const ovc_config& cfg, std::uint64_t seed,
     Upload(blk->alpha, src.Get(prefix + ".snake1.alpha", {1, channels, 1}, id, 0.1, true));
     const auto w = src.Get(prefix + ".conv_t1.weight", {channels, out, 2 * stride}, id + 1,
                            1.0 / std::sqrt(2.0 * channels));
-    Upload(blk->w, UpsampleLayout(w, channels, out, stride));
+    UploadConv(blk->w, UpsampleLayout(w, channels, out, stride), stride, 2, channels, out);
     Upload(blk->b, src.Get(prefix + ".conv_t1.bias", {out}, id + 2, 0.01));
     for (int u = 0; u < 3; ++u) {
       const std::string name = prefix + ".res_unit" + std::to_string(u + 1);
@@ -288,10 +289,9 @@ void CodecEngine::RunConv(const Conv& c, const float* x, int length, float* y, f
   p.phases = 1;
   p.positions = length;
   p.out_stride = 1;
-  p.accumulate = accumulate ? 1 : 0;
-  const int pad = (c.taps - 1) * c.dilation / 2;
-  for (int k = 0; k < c.taps; ++k)
-    p.offsets[0][k] = k * c.dilation - pad;
+  p.residual = accumulate ? y : nullptr;
+  p.dilation = c.dilation;
+  p.first[0] = -((c.taps - 1) * c.dilation / 2);
   const double flops = 2.0 * c.out * static_cast<double>(length) * c.in * c.taps;
   const double outputs = (y != nullptr ? 1.0 : 0.0) + (y_act != nullptr ? 1.0 : 0.0) +
                          (accumulate ? 1.0 : 0.0);
@@ -356,9 +356,8 @@ void CodecEngine::Enqueue(const std::int32_t* codes, std::int64_t frames, float*
     p.positions = length;
     p.out_stride = blk.stride;
     const UpsampleTaps u = Phases(blk.stride);
-    for (int ph = 0; ph < blk.stride; ++ph)
-      for (int k = 0; k < 2; ++k)
-        p.offsets[ph][k] = u.offsets[ph][k];
+    p.dilation = 1;
+    std::copy(u.first, u.first + kConvMaxPhases, p.first);
     run("codec_upsample", 2.0 * blk.out * double(length) * blk.stride * blk.in * 2,
         4.0 * length * (blk.in + 2.0 * blk.out * blk.stride) +
             4.0 * 2 * blk.stride * blk.in * blk.out,
@@ -561,8 +560,10 @@ int ovc_op_conv1d(const float* x, int64_t in, int64_t length, const float* alpha
                  "bad shape");
     const int I = static_cast<int>(in), O = static_cast<int>(out), K = static_cast<int>(kernel);
     const std::vector<float> host(w, w + static_cast<std::size_t>(O) * I * K);
-    ovg::DeviceBuffer<float> wd, bd;
-    ovg::Upload(wd, ovg::ConvLayout(host, O, I, K));
+    ovg::Require(K <= ovg::kConvMaxTaps, "1 to 7 taps");
+    ovg::DeviceBuffer<ovg::ConvUnit> wd;
+    ovg::DeviceBuffer<float> bd;
+    ovg::UploadConv(wd, ovg::ConvLayout(host, O, I, K), 1, K, I, O);
     ovg::Upload(bd, std::vector<float>(b, b + O));
     ovg::ConvParams p{};
     p.x = x;
@@ -578,11 +579,9 @@ int ovc_op_conv1d(const float* x, int64_t in, int64_t length, const float* alpha
     p.phases = 1;
     p.positions = static_cast<int>(length);
     p.out_stride = 1;
-    p.accumulate = accumulate ? 1 : 0;
-    const int pad = (K - 1) * static_cast<int>(dilation) / 2;
-    ovg::Require(K <= ovg::kConvMaxTaps, "1 to 7 taps");
-    for (int k = 0; k < K; ++k)
-      p.offsets[0][k] = k * static_cast<int>(dilation) - pad;
+    p.residual = accumulate ? y : nullptr;
+    p.dilation = static_cast<int>(dilation);
+    p.first[0] = -((K - 1) * static_cast<int>(dilation) / 2);
     auto s = static_cast<hipStream_t>(stream);
     ovg::LaunchConv(p, s);
     ovg::Check(hipStreamSynchronize(s), "conv1d");
@@ -602,8 +601,9 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length, const fl
                  "bad shape");
     const int I = static_cast<int>(in), O = static_cast<int>(out), S = static_cast<int>(stride);
     const std::vector<float> host(w, w + static_cast<std::size_t>(I) * O * 2 * S);
-    ovg::DeviceBuffer<float> wd, bd;
-    ovg::Upload(wd, ovg::UpsampleLayout(host, I, O, S));
+    ovg::DeviceBuffer<ovg::ConvUnit> wd;
+    ovg::DeviceBuffer<float> bd;
+    ovg::UploadConv(wd, ovg::UpsampleLayout(host, I, O, S), S, 2, I, O);
     ovg::Upload(bd, std::vector<float>(b, b + O));
     ovg::ConvParams p{};
     p.x = x;
@@ -620,9 +620,8 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length, const fl
     p.positions = static_cast<int>(length);
     p.out_stride = S;
     const ovg::UpsampleTaps u = ovg::Phases(S);
-    for (int ph = 0; ph < S; ++ph)
-      for (int k = 0; k < 2; ++k)
-        p.offsets[ph][k] = u.offsets[ph][k];
+    p.dilation = 1;
+    std::copy(u.first, u.first + ovg::kConvMaxPhases, p.first);
     auto s = static_cast<hipStream_t>(stream);
     ovg::LaunchConv(p, s);
     ovg::Check(hipStreamSynchronize(s), "conv_transpose1d");

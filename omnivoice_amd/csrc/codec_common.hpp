@@ -17,6 +17,7 @@
 
 #include "../../include/omnivoice_mi355x.h"
 #include "checkpoint.hpp"
+#include "codec.hpp"
 #include "device.hpp"
 #include "host.hpp"
 
@@ -70,9 +71,22 @@ void Upload(DeviceBuffer<T>& buffer, const std::vector<T>& host) {
   Check(hipDeviceSynchronize(), "upload codec weights");
 }
 
+// Convolution weights [lead][taps][in][out] as the kernel's operands.
+inline void UploadConv(DeviceBuffer<ConvUnit>& buffer, const std::vector<float>& host, int lead,
+                       int taps, int in, int out) {
+  Require(host.size() == static_cast<std::size_t>(lead) * taps * in * out,
+          "conv weights: bad size");
+  DeviceBuffer<float> staging;
+  Upload(staging, host);
+  buffer.Reserve(ConvWeightUnits(lead, taps, in, out));
+  LaunchPackConvWeights(staging.get(), lead, taps, in, out, buffer.get(), nullptr);
+  Check(hipGetLastError(), "conv weights");
+  Check(hipStreamSynchronize(nullptr), "conv weights");
+}
+
 // Conv1d weights [out][in][kernel] -> [kernel][in][out]. With kernel 1 and
-// in = channels x taps this is also the layout of a convolution run over
-// im2col columns: [channels x taps][out].
+// in = channels x taps this is also the layout of a convolution run as
+// one tap over channels x taps inputs: [channels x taps][out].
 inline std::vector<float> ConvLayout(const std::vector<float>& w, int out, int in, int kernel) {
   std::vector<float> r(w.size());
   for (int o = 0; o < out; ++o)

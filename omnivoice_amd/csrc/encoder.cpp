@@ -10,7 +10,8 @@
 // hidden states included ([width][steps]), so that every GEMM-shaped layer
 // is a convolution on the fp32 matrix cores (codec_kernels.hip):
 //  * a linear layer is a one-tap convolution;
-//  * a strided, long or grouped convolution runs over im2col columns;
+//  * a strided, long or grouped convolution reads its input through a strided
+//    window (ConvParams::view_kernel), a one-tap convolution of channels x taps;
 //  * attention is one kernel per layer over the heads' [dims][steps]
 //    projections (encoder_kernels.hip);
 //  * GELU, ELU and Snake are applied by the epilogue of the producing
@@ -73,22 +74,24 @@ constexpr std::int64_t kPartialFloats = std::int64_t{8} << 20;  // 32 MiB
 //   quantizer.quantizers.q.codebook.embed, project_out: the decoder's ids
 // (LayerNorm weights carry the offset 1).
 
-// A linear map on the matrix cores: w [in][out] (the im2col layout for a
-// convolution), bias [out] or none.
+// A linear map on the matrix cores: one tap over in = channels x kernel
+// inputs, bias [out] or none.
 struct Dense {
-  DeviceBuffer<float> w, b;
-  int in = 0, out = 0;
+  DeviceBuffer<ConvUnit> w;
+  DeviceBuffer<float> b;
+  int in = 0, out = 0, kernel = 1;
   bool bias = false;
 };
 
 void MakeDense(const std::vector<float>& w, const std::vector<float>* b, int out, int in,
                int kernel, Dense* d) {
-  Upload(d->w, ConvLayout(w, out, in * kernel, 1));
+  UploadConv(d->w, ConvLayout(w, out, in * kernel, 1), 1, 1, in * kernel, out);
   d->bias = b != nullptr;
   if (b != nullptr)
     Upload(d->b, *b);
   d->in = in * kernel;
   d->out = out;
+  d->kernel = kernel;
 }
 
 struct Layer {
@@ -96,7 +99,8 @@ struct Layer {
   DeviceBuffer<float> ln_w, ln_b, fln_w, fln_b;
 };
 struct Conv7 {
-  DeviceBuffer<float> w, b;  // [7][in][out], [out]
+  DeviceBuffer<ConvUnit> w;
+  DeviceBuffer<float> b;  // [out]
   int in = 0, out = 0, dilation = 1;
 };
 struct Unit {
@@ -146,8 +150,8 @@ class EncoderEngine {
   void Reserve(const Plan& plan);
   void Enqueue(const float* samples, const Plan& plan, std::int32_t* codes, hipStream_t stream,
                Profiler* prof);
-  // y = pre(W x + b) (or y += ...), y_act = out_act(...), over `positions`
-  // columns; `batches` independent maps with the given strides.
+  // y = pre(W x + b) (+ y), y_act = out_act(...), over `positions` columns.
+  // With len_in, x is [channels][len_in] read at position x stride + tap - pad.
   struct Gemm {
     const Dense* d = nullptr;
     const float* x = nullptr;
@@ -156,10 +160,9 @@ class EncoderEngine {
     const float* alpha_out = nullptr;
     int positions = 0, pre_act = kActNone, out_act = kActNone;
     bool accumulate = false;
+    int len_in = 0, stride = 1, pad = 0, in_act = kActNone;
   };
   void RunGemm(const Gemm& g, hipStream_t stream, Profiler* prof, const char* name);
-  void RunIm2col(const float* x, int channels, int len_in, int kernel, int stride, int pad,
-                 int positions, int act, hipStream_t stream, Profiler* prof, const char* name);
   void RunConv7(const Conv7& c, const float* x, int length, float* y, float* y_act,
                 const float* alpha_out, bool accumulate, hipStream_t stream, Profiler* prof,
                 const char* name);
@@ -173,19 +176,19 @@ class EncoderEngine {
   // HuBERT
   std::vector<std::unique_ptr<Dense>> features_;
   DeviceBuffer<float> gn_w_, gn_b_, proj_ln_w_, proj_ln_b_, enc_ln_w_, enc_ln_b_;
-  Dense projection_, position_;  // position_: [groups][in_g K][out_g]
+  Dense projection_, position_;  // position_: a lead per group
   std::vector<std::unique_ptr<Layer>> layers_;
   // semantic encoder
   Dense sem_in_, sem_c1_[2][2], sem_c2_[2][2], sem_block_[2];
   // DAC encoder
-  Conv7 ac_in_;
+  Dense ac_in_;
   std::vector<std::unique_ptr<Block>> blocks_;
   DeviceBuffer<float> ac_alpha_;
   Dense ac_out_, fc_;
   std::vector<std::unique_ptr<Stage>> stages_;
   DeviceBuffer<RvqStage> stage_list_;
   // work buffers
-  DeviceBuffer<float> samples_, wave_, fa_, fb_, cols_, tmp_, h_, qkv_, ctx_, ff_;
+  DeviceBuffer<float> samples_, wave_, fa_, fb_, tmp_, h_, qkv_, ctx_, ff_;
   DeviceBuffer<double> sum_;
   DeviceBuffer<std::uint16_t> heads_;  // the attention's operands
   // Split-K workspace of the thin GEMMs (HuBERT at short lengths, the
@@ -286,10 +289,11 @@ EncoderEngine::EncoderEngine(const ovc_encoder_config& cfg, std::uint64_t seed,
           w[(static_cast<std::size_t>(grp) * Wg * K + static_cast<std::size_t>(i) * K + k) * Wg +
             oo] = static_cast<float>(g[k] * v[src_at] / std::sqrt(norm[k]));
         }
-    Upload(position_.w, w);
+    UploadConv(position_.w, w, G, 1, Wg * K, Wg);
     Upload(position_.b, src.Get(p + "bias", {W}, 2018, 0.01));
     position_.bias = true;
     position_.in = Wg * K;
+    position_.kernel = K;
     position_.out = Wg;
   }
   Upload(enc_ln_w_, src.Get("semantic_model.encoder.layer_norm.weight", {W}, 2019, 0.1, false,
@@ -348,10 +352,8 @@ EncoderEngine::EncoderEngine(const ovc_encoder_config& cfg, std::uint64_t seed,
   const int ce = static_cast<int>(cfg.enc_channels);
   {
     const auto w = src.Get("acoustic_encoder.conv1.weight", {ce, 1, 7}, 2500, 1.0 / std::sqrt(7.0));
-    Upload(ac_in_.w, ConvLayout(w, ce, 1, 7));
-    Upload(ac_in_.b, src.Get("acoustic_encoder.conv1.bias", {ce}, 2501, 0.01));
-    ac_in_.in = 1;
-    ac_in_.out = ce;
+    const auto b = src.Get("acoustic_encoder.conv1.bias", {ce}, 2501, 0.01);
+    MakeDense(w, &b, ce, 1, 7, &ac_in_);
   }
   int ch = ce;
   for (int i = 0; i < cfg.blocks; ++i) {
@@ -368,7 +370,7 @@ EncoderEngine::EncoderEngine(const ovc_encoder_config& cfg, std::uint64_t seed,
       Upload(unit.alpha1, src.Get(name + ".snake1.alpha", {1, ch, 1}, uid, 0.1, true));
       const auto w1 = src.Get(name + ".conv1.weight", {ch, ch, 7}, uid + 1,
                               1.0 / std::sqrt(7.0 * ch));
-      Upload(unit.conv1.w, ConvLayout(w1, ch, ch, 7));
+      UploadConv(unit.conv1.w, ConvLayout(w1, ch, ch, 7), 1, 7, ch, ch);
       Upload(unit.conv1.b, src.Get(name + ".conv1.bias", {ch}, uid + 2, 0.01));
       unit.conv1.in = unit.conv1.out = ch;
       unit.conv1.dilation = kDilations[u];
@@ -478,6 +480,7 @@ Plan EncoderEngine::MakePlan(int64_t length) const {
 
 void EncoderEngine::Reserve(const Plan& p) {
   const int64_t W = W_, T = p.steps, F = p.frames;
+  // cols: the largest convolution's channels x taps x positions, a bound only.
   int64_t feat = 0, cols = 0;
   int64_t in = 1, len = p.resampled + 2 * kWavePad;
   for (int i = 0; i < cfg_.feature_layers; ++i) {
@@ -511,7 +514,6 @@ void EncoderEngine::Reserve(const Plan& p) {
   grow(wave_, p.resampled + 2 * kWavePad);
   grow(fa_, feat);
   grow(fb_, feat);
-  grow(cols_, cols);
   grow(tmp_, hid);
   grow(h_, W * T);
   grow(qkv_, 3 * W * T);
@@ -543,14 +545,21 @@ void EncoderEngine::RunGemm(const Gemm& g, hipStream_t stream, Profiler* prof,
   p.y_act = g.y_act;
   p.alpha_out = g.alpha_out;
   p.cin = g.d->in;
-  p.len_in = g.positions;
+  p.len_in = g.len_in > 0 ? g.len_in : g.positions;
   p.cout = g.d->out;
   p.len_out = g.positions;
   p.taps = 1;
   p.phases = 1;
   p.positions = g.positions;
   p.out_stride = 1;
-  p.accumulate = g.accumulate ? 1 : 0;
+  if (g.len_in > 0) {
+    p.view_kernel = g.d->kernel;
+    p.view_stride = g.stride;
+    p.channels = g.d->in / g.d->kernel;
+    p.first[0] = -g.pad;
+  }
+  p.in_act = g.in_act;
+  p.residual = g.accumulate ? g.y : nullptr;
   p.pre_act = g.pre_act;
   p.out_act = g.out_act;
   p.partial = partial_.get();
@@ -558,23 +567,11 @@ void EncoderEngine::RunGemm(const Gemm& g, hipStream_t stream, Profiler* prof,
   const double flops = 2.0 * p.cin * p.cout * static_cast<double>(p.positions);
   const double outs = (g.y != nullptr) + (g.y_act != nullptr) + (g.accumulate ? 1 : 0);
   const double bytes =
-      4.0 * (static_cast<double>(p.cin) * p.positions + outs * p.cout * p.positions +
+      4.0 * (static_cast<double>(p.cin / g.d->kernel) * p.len_in + outs * p.cout * p.positions +
              static_cast<double>(p.cin) * p.cout);
   auto launch = [&] { LaunchConv(p, stream); };
   if (prof != nullptr)
     prof->Run(name, flops, bytes, launch);
-  else
-    launch();
-}
-
-void EncoderEngine::RunIm2col(const float* x, int channels, int len_in, int kernel, int stride,
-                              int pad, int positions, int act, hipStream_t stream,
-                              Profiler* prof, const char* name) {
-  Im2colParams p{x, cols_.get(), channels, len_in, kernel, stride, 1, pad, positions, act};
-  const double bytes = 8.0 * channels * static_cast<double>(kernel) * positions;
-  auto launch = [&] { LaunchIm2col(p, stream); };
-  if (prof != nullptr)
-    prof->Run(name, 0.0, bytes, launch);
   else
     launch();
 }
@@ -597,11 +594,11 @@ void EncoderEngine::RunConv7(const Conv7& c, const float* x, int length, float* 
   p.phases = 1;
   p.positions = length;
   p.out_stride = 1;
-  p.accumulate = accumulate ? 1 : 0;
+  p.residual = accumulate ? y : nullptr;
   p.partial = partial_.get();
   p.partial_capacity = kPartialFloats;
-  for (int k = 0; k < 7; ++k)
-    p.offsets[0][k] = (k - 3) * c.dilation;
+  p.dilation = c.dilation;
+  p.first[0] = -3 * c.dilation;
   const double flops = 2.0 * c.out * static_cast<double>(length) * c.in * 7;
   const double outs = (y != nullptr) + (y_act != nullptr) + (accumulate ? 1 : 0);
   const double bytes = 4.0 * length * (c.in + c.out * outs) + 28.0 * c.in * c.out;
@@ -634,12 +631,13 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
   float* a = fa_.get();
   float* b = fb_.get();
   for (int i = 0; i < cfg_.feature_layers; ++i) {
-    const int k = static_cast<int>(cfg_.conv_kernel[i]), s = static_cast<int>(cfg_.conv_stride[i]);
+    const int s = static_cast<int>(cfg_.conv_stride[i]);
     const int out_len = static_cast<int>(plan.features[i]);
-    RunIm2col(x, in, len, k, s, 0, out_len, kActNone, stream, prof, "enc_feature_im2col");
     Gemm g;
     g.d = features_[i].get();
-    g.x = cols_.get();
+    g.x = x;
+    g.len_in = len;
+    g.stride = s;
     g.y = b;
     g.positions = out_len;
     g.pre_act = i == 0 ? kActNone : kActGelu;
@@ -671,16 +669,21 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
   }
   {
     // Grouped positional convolution: padding K / 2, the first T outputs,
-    // GELU, added to the states.
+    // GELU, added to the states; every work-group reads its neighbours'
+    // states, so the sum goes to another buffer.
     const int K = static_cast<int>(cfg_.pos_kernel), G = static_cast<int>(cfg_.pos_groups);
     const int Wg = W / G;
-    RunIm2col(h_.get(), W, T, K, 1, K / 2, T, kActNone, stream, prof, "enc_pos_im2col");
     ConvParams p{};
-    p.x = cols_.get();
+    p.x = h_.get();
     p.w = position_.w.get();
     p.bias = position_.b.get();
-    p.y = h_.get();
+    p.y = tmp_.get();
+    p.residual = h_.get();
     p.cin = Wg * K;
+    p.channels = Wg;
+    p.view_kernel = K;
+    p.view_stride = 1;
+    p.first[0] = -(K / 2);
     p.len_in = T;
     p.cout = Wg;
     p.len_out = T;
@@ -688,20 +691,18 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
     p.phases = 1;
     p.positions = T;
     p.out_stride = 1;
-    p.accumulate = 1;
     p.pre_act = kActGelu;
     p.batches = G;
     p.partial = partial_.get();
     p.partial_capacity = kPartialFloats;
-    p.x_batch = static_cast<int64_t>(Wg) * K * T;
-    p.w_batch = static_cast<int64_t>(Wg) * K * Wg;
+    p.x_batch = static_cast<int64_t>(Wg) * T;
     p.b_batch = Wg;
     p.y_batch = static_cast<int64_t>(Wg) * T;
     run("enc_pos_conv", 2.0 * W * Wg * K * static_cast<double>(T),
-        4.0 * (static_cast<double>(W) * K * T + 2.0 * W * T + static_cast<double>(W) * Wg * K),
+        4.0 * (3.0 * W * T + static_cast<double>(W) * Wg * K),
         [&] { LaunchConv(p, stream); });
   }
-  norm(h_.get(), h_.get(), enc_ln_w_, enc_ln_b_, W, 1);
+  norm(tmp_.get(), h_.get(), enc_ln_w_, enc_ln_b_, W, 1);
   for (const auto& layer : layers_) {
     const Layer& ly = *layer;
     Gemm g;
@@ -749,62 +750,75 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
   // ---- semantic encoder (codec_encoder.cpp:400-416)
   const int lat = static_cast<int>(cfg_.latent);
   float* semantic_rows = joint_.get() + static_cast<std::size_t>(lat) * F;
-  RunIm2col(sem_.get(), W, F, 3, 1, 1, F, kActNone, stream, prof, "enc_sem_im2col");
-  {
+  float *st = st_.get(), *t1 = t1_.get();
+  auto conv3 = [&](const Dense& d, const float* from, int in_act) {
     Gemm g;
-    g.d = &sem_in_;
-    g.x = cols_.get();
-    g.y = st_.get();
+    g.d = &d;
+    g.x = from;
+    g.len_in = F;
+    g.pad = 1;
+    g.in_act = in_act;
     g.positions = F;
+    return g;
+  };
+  {
+    Gemm g = conv3(sem_in_, sem_.get(), kActNone);
+    g.y = st;
     RunGemm(g, stream, prof, "enc_sem_conv");
   }
   for (int bl = 0; bl < 2; ++bl) {
     for (int u = 0; u < 2; ++u) {
-      RunIm2col(st_.get(), W, F, 3, 1, 1, F, kActElu, stream, prof, "enc_sem_im2col");
-      Gemm g;
-      g.d = &sem_c1_[bl][u];
-      g.x = cols_.get();
-      g.y_act = t1_.get();
+      Gemm g = conv3(sem_c1_[bl][u], st, kActElu);
+      g.y_act = t1;
       g.out_act = kActElu;
-      g.positions = F;
       RunGemm(g, stream, prof, "enc_sem_conv");
       g = Gemm();
       g.d = &sem_c2_[bl][u];
-      g.x = t1_.get();
-      g.y = st_.get();
+      g.x = t1;
+      g.y = st;
       g.positions = F;
       g.accumulate = true;
       RunGemm(g, stream, prof, "enc_sem_conv");
     }
-    RunIm2col(st_.get(), W, F, 3, 1, 1, F, kActNone, stream, prof, "enc_sem_im2col");
-    Gemm g;
-    g.d = &sem_block_[bl];
-    g.x = cols_.get();
-    g.y = bl == 1 ? semantic_rows : st_.get();
-    g.positions = F;
+    Gemm g = conv3(sem_block_[bl], st, kActNone);
+    g.y = bl == 1 ? semantic_rows : t1;
     RunGemm(g, stream, prof, "enc_sem_conv");
+    std::swap(st, t1);
   }
 
   // ---- DAC encoder on the 24 kHz samples (codec_encoder.cpp:417-452).
   // xa holds snake(x) with the alpha of whatever reads it next, ya the
-  // residual branch's snake(conv1(...)).
+  // residual branch's snake(conv1(...)); a downsampling layer reads one and
+  // writes the other.
+  float *xa = xa_.get(), *ya = ya_.get();
   auto first_alpha = [&](std::size_t bi) {
     return bi < blocks_.size() ? blocks_[bi]->units[0].alpha1.get() : ac_alpha_.get();
   };
-  RunConv7(ac_in_, samples, L, x_.get(), xa_.get(), first_alpha(0), false, stream, prof,
-           "enc_dac_conv_in");
+  {
+    Gemm g;
+    g.d = &ac_in_;
+    g.x = samples;
+    g.len_in = L;
+    g.pad = 3;
+    g.y = x_.get();
+    g.y_act = xa;
+    g.out_act = kActSnake;
+    g.alpha_out = first_alpha(0);
+    g.positions = L;
+    RunGemm(g, stream, prof, "enc_dac_conv_in");
+  }
   int cur = L;
   for (std::size_t bi = 0; bi < blocks_.size(); ++bi) {
     const Block& blk = *blocks_[bi];
     for (int u = 0; u < 3; ++u) {
       const Unit& unit = blk.units[u];
-      RunConv7(unit.conv1, xa_.get(), cur, nullptr, ya_.get(), unit.alpha2.get(), false, stream,
+      RunConv7(unit.conv1, xa, cur, nullptr, ya, unit.alpha2.get(), false, stream,
                prof, "enc_dac_res_conv7");
       Gemm g;
       g.d = &unit.conv2;
-      g.x = ya_.get();
+      g.x = ya;
       g.y = x_.get();
-      g.y_act = xa_.get();
+      g.y_act = xa;
       g.out_act = kActSnake;
       g.alpha_out = u < 2 ? blk.units[u + 1].alpha1.get() : blk.alpha.get();
       g.positions = cur;
@@ -812,25 +826,27 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
       RunGemm(g, stream, prof, "enc_dac_res_conv1");
     }
     const int s = blk.stride, out_len = static_cast<int>(plan.acoustic[bi]);
-    RunIm2col(xa_.get(), blk.channels, cur, 2 * s, s, (s + 1) / 2, out_len, kActNone, stream,
-              prof, "enc_dac_im2col");
     Gemm g;
     g.d = &blk.down;
-    g.x = cols_.get();
+    g.x = xa;
+    g.len_in = cur;
+    g.stride = s;
+    g.pad = (s + 1) / 2;
     g.y = x_.get();
-    g.y_act = xa_.get();
+    g.y_act = ya;
     g.out_act = kActSnake;
     g.alpha_out = first_alpha(bi + 1);
     g.positions = out_len;
     RunGemm(g, stream, prof, "enc_dac_down");
+    std::swap(xa, ya);
     cur = out_len;
   }
-  const int chf = static_cast<int>(cfg_.enc_channels << cfg_.blocks);
-  RunIm2col(xa_.get(), chf, cur, 3, 1, 1, F, kActNone, stream, prof, "enc_dac_im2col");
   {
     Gemm g;
     g.d = &ac_out_;
-    g.x = cols_.get();
+    g.x = xa;
+    g.len_in = cur;
+    g.pad = 1;
     g.y = joint_.get();
     g.positions = F;
     RunGemm(g, stream, prof, "enc_dac_out");

@@ -22,16 +22,6 @@ struct ResampleParams {
 };
 void LaunchResample(const ResampleParams& p, hipStream_t stream);
 
-// Columns of a strided, dilated, padded convolution:
-// y[c kernel + j][t] = act(x[c][t stride + j dilation - pad]), zero outside
-// [0, len_in); act the identity or ELU (kActElu).
-struct Im2colParams {
-  const float* x;  // [channels][len_in]
-  float* y;        // [channels * kernel][positions]
-  int channels, len_in, kernel, stride, dilation, pad, positions, act;
-};
-void LaunchIm2col(const Im2colParams& p, hipStream_t stream);
-
 // GroupNorm with one group per channel (statistics over the row), affine,
 // then GELU, in place: x [channels][length].
 void LaunchGroupNormGelu(float* x, const float* w, const float* b, int channels, int length,

@@ -29,7 +29,6 @@ constexpr int kThreads = 256;
 __device__ __forceinline__ float Gelu(float v) {
   return 0.5F * v * (1.0F + erff(v * 0.70710678118654752F));
 }
-__device__ __forceinline__ float Elu(float v) { return v > 0.0F ? v : expm1f(v); }
 
 __global__ __launch_bounds__(kThreads) void ResampleKernel(ResampleParams p) {
   const int total = p.out_length + 2 * p.pad;
@@ -47,25 +46,6 @@ __global__ __launch_bounds__(kThreads) void ResampleKernel(ResampleParams p) {
       out = static_cast<float>(sum);
     }
     p.y[i] = out;
-  }
-}
-
-__global__ __launch_bounds__(kThreads) void Im2colKernel(Im2colParams p) {
-  const size_t total = static_cast<size_t>(p.channels) * p.kernel * p.positions;
-  for (size_t e = static_cast<size_t>(blockIdx.x) * kThreads + threadIdx.x; e < total;
-       e += static_cast<size_t>(gridDim.x) * kThreads) {
-    const int t = static_cast<int>(e % p.positions);
-    const int r = static_cast<int>(e / p.positions);
-    const int j = r % p.kernel;
-    const int c = r / p.kernel;
-    const int s = t * p.stride + j * p.dilation - p.pad;
-    float v = 0.0F;
-    if (s >= 0 && s < p.len_in) {
-      v = p.x[static_cast<size_t>(c) * p.len_in + s];
-      if (p.act == kActElu)
-        v = Elu(v);
-    }
-    p.y[e] = v;
   }
 }
 
@@ -600,16 +580,6 @@ void LaunchResample(const ResampleParams& p, hipStream_t stream) {
           "resample: bad shape");
   Dispatch(ResampleKernel, dim3(Blocks(static_cast<size_t>(p.out_length) + 2 * p.pad)),
            dim3(kThreads), 0, stream, true, true, p);
-}
-
-void LaunchIm2col(const Im2colParams& p, hipStream_t stream) {
-  Require(p.x && p.y, "im2col: null pointer");
-  Require(p.channels >= 1 && p.len_in >= 1 && p.kernel >= 1 && p.stride >= 1 &&
-              p.dilation >= 1 && p.pad >= 0 && p.positions >= 1,
-          "im2col: bad shape");
-  Require(p.act == kActNone || p.act == kActElu, "im2col: bad activation");
-  const size_t total = static_cast<size_t>(p.channels) * p.kernel * p.positions;
-  Dispatch(Im2colKernel, dim3(Blocks(total)), dim3(kThreads), 0, stream, true, true, p);
 }
 
 void LaunchGroupNormGelu(float* x, const float* w, const float* b, int channels, int length,

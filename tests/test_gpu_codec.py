@@ -71,6 +71,43 @@ def test_conv1d_matches_oracle(cin, cout, length, kernel, dilation, snake, accum
     close(y.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("cin,cout,length,kernel,dilation", [
+    (1, 1, 1, 7, 10), (31, 32, 255, 7, 9), (32, 31, 257, 7, 10), (33, 33, 129, 7, 1),
+    (64, 64, 127, 1, 1), (65, 65, 64, 1, 1), (63, 129, 65, 7, 3), (130, 200, 63, 1, 1),
+    (97, 128, 16500, 7, 9), (40, 130, 16400, 1, 1), (17, 16, 300, 2, 1)])
+def test_conv1d_tile_edges(cin, cout, length, kernel, dilation):
+    """Edges of the tiles, chunks and windows against 64 bits. Bound: every operand is kept to
+    2^-24 and what is left out of a product is below 2^-23 of it; each 16-deep product rounds
+    its two sums once, five of six of them small: K / 8 + 8 roundings of 2^-24 of sum |w x|."""
+    rng = np.random.default_rng(cin + cout + length)
+    x = rng.standard_normal((cin, length)).astype(np.float32)
+    w = (rng.standard_normal((cout, cin, kernel)) / math.sqrt(cin * kernel)).astype(np.float32)
+    b = rng.standard_normal(cout).astype(np.float32)
+    y = dev(np.zeros((cout, length)))
+    ov.op_conv1d(dev(x), w, b, y, dilation=dilation)
+    pad = (kernel - 1) * dilation // 2
+    xp = np.pad(x.astype(np.float64), ((0, 0), (pad, kernel * dilation)))
+    want, size = b.astype(np.float64)[:, None], np.abs(b)[:, None].astype(np.float64)
+    for k in range(kernel):
+        at = xp[:, k * dilation:k * dilation + length]
+        want = want + w[:, :, k].astype(np.float64) @ at
+        size = size + np.abs(w[:, :, k]).astype(np.float64) @ np.abs(at)
+    assert (np.abs(y.cpu().numpy() - want) <= (cin * kernel / 8 + 8) * 2.0 ** -24 * size).all()
+
+
+def test_conv1d_keeps_infinities():
+    """An infinite input makes its outputs infinite, not NaN; NaN stays where it reaches."""
+    x = np.ones((32, 200), dtype=np.float32)
+    x[3, 50], x[5, 120] = np.inf, np.nan
+    w = np.full((32, 32, 7), 0.5, dtype=np.float32)
+    y = dev(np.zeros((32, 200)))
+    ov.op_conv1d(dev(x), w, np.zeros(32, np.float32), y)
+    got = y.cpu().numpy()
+    assert np.isposinf(got[:, 47:54]).all() and np.isnan(got[:, 117:124]).all()
+    rest = np.delete(got, [*range(47, 54), *range(117, 124)], axis=1)
+    assert np.isfinite(rest).all()
+
+
 @pytest.mark.parametrize("cin,cout,length,stride,snake", [
     (64, 32, 40, 8, True), (32, 16, 33, 5, True), (128, 64, 70, 4, False),
     (16, 8, 9, 2, True), (48, 24, 31, 3, True), (1024, 512, 25, 8, True),

@@ -140,6 +140,8 @@ class CodecEngine {
   void RunConv(const Conv& c, const float* x, int length, float* y, float* y_act,
                const float* alpha_out, bool accumulate, hipStream_t stream, Profiler* prof,
                const char* name);
+  void RunUnit(const Unit& unit, const float* x, int length, float* y_act,
+               const float* alpha_out, hipStream_t stream, Profiler* prof);
 
   ovc_config cfg_;
   std::int64_t hop_ = 1;
@@ -288,7 +290,6 @@ void CodecEngine::RunConv(const Conv& c, const float* x, int length, float* y, f
   p.taps = c.taps;
   p.phases = 1;
   p.positions = length;
-  p.out_stride = 1;
   p.residual = accumulate ? y : nullptr;
   p.dilation = c.dilation;
   p.first[0] = -((c.taps - 1) * c.dilation / 2);
@@ -299,6 +300,35 @@ void CodecEngine::RunConv(const Conv& c, const float* x, int length, float* y, f
   auto launch = [&] { LaunchConv(p, stream); };
   if (prof != nullptr)
     prof->Run(name, flops, bytes, launch);
+  else
+    launch();
+}
+
+// A whole residual unit: x_ += conv2(snake(conv1(x))), y_act its Snake.
+void CodecEngine::RunUnit(const Unit& unit, const float* x, int length, float* y_act,
+                          const float* alpha_out, hipStream_t stream, Profiler* prof) {
+  const Conv& c = unit.conv1;
+  ConvParams p{};
+  p.x = x;
+  p.w = c.w.get();
+  p.bias = c.b.get();
+  p.w2 = unit.conv2.w.get();
+  p.bias2 = unit.conv2.b.get();
+  p.alpha_mid = unit.alpha2.get();
+  p.residual = p.y = x_.get();
+  p.y_act = y_act;
+  p.alpha_out = alpha_out;
+  p.cin = p.cout = c.out;
+  p.len_in = p.len_out = p.positions = length;
+  p.taps = c.taps;
+  p.phases = 1;
+  p.dilation = c.dilation;
+  p.first[0] = -((c.taps - 1) * c.dilation / 2);
+  const double flops = 2.0 * c.out * static_cast<double>(length) * c.out * (c.taps + 1);
+  const double bytes = 16.0 * length * c.out + 4.0 * (c.taps + 1) * c.out * c.out;
+  auto launch = [&] { LaunchConv(p, stream); };
+  if (prof != nullptr)
+    prof->Run("codec_res_unit", flops, bytes, launch);
   else
     launch();
 }
@@ -354,7 +384,6 @@ void CodecEngine::Enqueue(const std::int32_t* codes, std::int64_t frames, float*
     p.taps = 2;
     p.phases = blk.stride;
     p.positions = length;
-    p.out_stride = blk.stride;
     const UpsampleTaps u = Phases(blk.stride);
     p.dilation = 1;
     std::copy(u.first, u.first + kConvMaxPhases, p.first);
@@ -370,6 +399,11 @@ void CodecEngine::Enqueue(const std::int32_t* codes, std::int64_t frames, float*
       const float* next_alpha = ui < 2 ? blk.units[ui + 1].alpha1.get()
                                 : bi + 1 < blocks_.size() ? blocks_[bi + 1]->alpha.get()
                                                           : final_alpha_.get();
+      if (blk.out <= kConvFusedChannels) {
+        RunUnit(unit, xa_[cur].get(), length, xa_[1 - cur].get(), next_alpha, stream, prof);
+        cur = 1 - cur;
+        continue;
+      }
       RunConv(unit.conv1, xa_[cur].get(), length, nullptr, ya_.get(), unit.alpha2.get(), false,
               stream, prof, "codec_res_conv7");
       RunConv(unit.conv2, ya_.get(), length, x_.get(), xa_[cur].get(), next_alpha, true, stream,
@@ -578,7 +612,6 @@ int ovc_op_conv1d(const float* x, int64_t in, int64_t length, const float* alpha
     p.taps = K;
     p.phases = 1;
     p.positions = static_cast<int>(length);
-    p.out_stride = 1;
     p.residual = accumulate ? y : nullptr;
     p.dilation = static_cast<int>(dilation);
     p.first[0] = -((K - 1) * static_cast<int>(dilation) / 2);
@@ -618,7 +651,6 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length, const fl
     p.taps = 2;
     p.phases = S;
     p.positions = static_cast<int>(length);
-    p.out_stride = S;
     const ovg::UpsampleTaps u = ovg::Phases(S);
     p.dilation = 1;
     std::copy(u.first, u.first + ovg::kConvMaxPhases, p.first);

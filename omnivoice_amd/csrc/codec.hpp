@@ -16,6 +16,9 @@ constexpr int kConvMaxPhases = 8;
 // dilation 9 spans 54 samples).
 constexpr int kConvMaxSpan = 64;
 
+// Largest residual unit that runs as one launch.
+constexpr int kConvFusedChannels = 128;
+
 // Activations a convolution's epilogue applies.
 enum ConvAct : int {
   kActNone = 0,
@@ -40,14 +43,17 @@ void LaunchPackConvWeights(const float* w, int lead, int taps, int cin, int cout
 // One float32 convolution as an implicit GEMM on the matrix cores:
 //   v[o][t] = pre(bias[o] + sum_{k, i} w[phase][k][i][o] *
 //                 act_in(x[i][m + first[phase] + k dilation]))
-//   y[o][t] = v (+ residual[o][t]), y_act[o][t] = out_act(y[o][t]),  t = m out_stride + phase
+//   y[o][t] = v (+ residual[o][t]), y_act[o][t] = out_act(y[o][t]),  t = m phases + phase
 // for output positions m < positions, with x = 0 outside [0, len_in), and
 // act_in the Snake activation of the channel's alpha (the identity when
 // alpha_in is null), then in_act. A Conv1d is one phase with first = -pad; a
 // ConvTranspose1d of stride s is s phases of two taps each (see the codec
 // engine). With view_kernel, x has `channels` channels and K index i stands
 // for x[i / view_kernel][m view_stride + first + i % view_kernel] (a strided
-// or long convolution of one tap, cin = channels x view_kernel). Either
+// or long convolution of one tap, cin = channels x view_kernel). With w2 the
+// launch is a residual unit of up to kConvFusedChannels channels: v passes
+// through the Snake of alpha_mid and the one-tap convolution w2, bias2 before
+// the residual (x is then neither y nor y_act). Either
 // output may be null; bias may be null (zero); residual may be y.
 // `batches` independent convolutions of the same shape run in one launch, the
 // pointers of batch b advanced by b times their batch strides, the weights by
@@ -57,12 +63,15 @@ struct ConvParams {
   const float* alpha_in;  // [cin] or null
   const ConvUnit* w;      // lead = batches x phases
   const float* bias;      // [cout] or null
+  const ConvUnit* w2;     // [cout][cout], or null
+  const float* bias2;     // [cout], with w2
+  const float* alpha_mid; // [cout], with w2
   const float* residual;  // [cout][len_out] or null
   float* y;               // [cout][len_out] or null
   float* y_act;           // [cout][len_out] or null
   const float* alpha_out; // [cout], with a Snake output activation
   int cin, len_in, cout, len_out;
-  int taps, dilation, phases, positions, out_stride;
+  int taps, dilation, phases, positions;
   int view_kernel, view_stride, channels;  // view_kernel 0: none
   int in_act;      // kActNone or kActElu
   int pre_act;     // kActNone or kActGelu

@@ -22,7 +22,7 @@ constexpr int kOutChunk = 32;  // input channels per chunk of the output conv
 
 // kernels/codec_kernels.hip:20-22 of the reference: v + sin^2(a v) / (a + 1e-9),
 // with 1 / (a + 1e-9) given. x = a v less its nearest multiple of pi (pi in
-// three parts; the first difference is exact, both terms being multiples of
+// two parts; the first difference is exact, both terms being multiples of
 // one unit and the difference below 2^24 of them), then the Taylor series of
 // the sine up to r^13, whose remainder at pi / 2 is 2^-30 of the sine: about
 // 18 operations where sinf has 40 and a branch. The term is at most 1 / |x|
@@ -33,7 +33,6 @@ __device__ __forceinline__ float Snake(float v, float a, float inverse) {
   const float n = rintf(x * 0.31830988618379067F);
   float r = fmaf(n, -3.1415927410125732F, x);
   r = fmaf(n, 8.7422776573475858e-8F, r);
-  r = fmaf(n, 3.4302490902798e-15F, r);
   const float u = r * r;
   float s = 1.0F / 6227020800.0F;
   s = fmaf(s, u, -1.0F / 39916800.0F);
@@ -68,6 +67,20 @@ __device__ __forceinline__ void Finish(const ConvParams& p, const float* bias,
     y_act[at] = p.out_act == kActElu ? Elu(v) : Snake(v, p.alpha_out[co], SnakeInverse(p.alpha_out[co]));
 }
 
+// Four floats at any 4-byte address.
+typedef float Unaligned4 __attribute__((ext_vector_type(4), aligned(4)));
+
+// The six products of a step's 32 x 32 block.
+__device__ __forceinline__ void Products(const uintx4* a, const uintx4* b, floatx16& main,
+                                         floatx16& low) {
+  low = MfmaBf16(a[0], b[2], low);
+  main = MfmaBf16(a[0], b[0], main);
+  low = MfmaBf16(a[2], b[0], low);
+  low = MfmaBf16(a[1], b[1], low);
+  low = MfmaBf16(a[0], b[1], low);
+  low = MfmaBf16(a[1], b[0], low);
+}
+
 // Work-group `id` of `count` to a tile such that each XCD (id % 8) has a run
 // of consecutive tiles.
 __device__ __forceinline__ int XcdTile(int id, int count) {
@@ -94,29 +107,60 @@ constexpr int TileChunk(int taps, int columns) { return taps == 1 && columns <= 
 // reads the window at its own shift. One barrier per chunk: two LDS buffers,
 // or one where there is one chunk.
 //
-// VIEW reads the input through a strided window: K index j is tap j % view_kernel of channel j /
-// view_kernel (an im2col that is never stored).
-template <int WM, int WN, int NT, int TAPS, int BUFS, bool VIEW>
-__global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
-  static_assert(WM * WN * 64 == kThreads, "four waves");
+// A residual unit's k1 convolution follows in the same work-group where one
+// tile holds every channel (FUSED): the k7 results, biased and through their
+// Snake, are split back into LDS as the second product's operand and never
+// see memory. A transposed convolution (kUp) gives each wave one phase of the
+// same 32 channels, so that the work-group's outputs are whole runs.
+//
+// VIEW reads the input through a strided window: K index j is tap j %
+// view_kernel of channel j / view_kernel (an im2col that is never stored).
+//
+// Bound by the matrix cores (their pipes 52-60 % busy at the 1.9 GHz this
+// work draws) at 128 channels and more; at 32 and 64 by them, the activations'
+// vector work and memory alike. At a 60 s signal: the k7 convolutions of 256
+// and 512 channels 195 TFLOP/s of float32 products (87 on the float32 matrix
+// cores), a residual unit of 128 / 64 / 32 channels 379 / 278 / 301 us where
+// its two launches took 492 / 329 / 397, the transposed convolutions 230 us
+// a launch where one phase per work-group, its outputs scattered, took 295.
+// Blocks multiplied two in turn, or the fused tiles' weights seven steps
+// ahead, cost the third wave per SIMD (379 -> 441, 407 us).
+enum ConvKind : int { kPlain, kView, kFused, kUp };
+
+template <int WM, int WN, int NT, int TAPS, int BUFS, ConvKind KIND>
+__global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
+  constexpr bool VIEW = KIND == kView, FUSED = KIND == kFused, UP = KIND == kUp;
   static_assert(!VIEW || TAPS == 1, "a view has its taps in K");
-  constexpr int BM = 32 * WM, BN = 32 * WN * NT;
-  constexpr int kMaxWidth = BN + (TAPS == 1 ? 0 : TAPS == 2 ? 1 : kConvMaxSpan);
+  static_assert(!UP || (TAPS == 2 && WN == 1), "a wave per phase");
+  constexpr int kT = 64 * WM * WN;
+  constexpr int S = UP ? WM : 1;  // output positions per position of the tile
+  constexpr int BM = UP ? 32 : 32 * WM, BN = 32 * WN * NT;
   constexpr int kChunk = TileChunk(TAPS, BN);
+  constexpr int kMaxWidth = BN + (TAPS == 1 ? 0 : UP ? 2 : TAPS == 2 ? 1 : kConvMaxSpan);
   constexpr int kMaxUnits = kChunk / 8 * kMaxWidth;
-  constexpr int kSlots = (kMaxUnits + kThreads - 1) / kThreads;
+  constexpr int kSlots = (kMaxUnits + kT - 1) / kT;
   constexpr int kSubs = kChunk / 16;
   constexpr int kSteps = kSubs * TAPS;  // of 16 channels, per chunk
   // Steps the weights are loaded ahead: a narrow tile's short steps and large
   // weights need more.
-  constexpr int kAhead = WM < 4 || NT == 4 ? 2 : TAPS == 7 ? 7 : 4;
+  constexpr int kAhead = NT == 4 || FUSED ? 2 : TAPS == 7 ? 7 : UP || WM == 4 ? 4 : 2;
   static_assert(kSteps % kAhead == 0, "weight registers");
-  __shared__ uintx4 xs[BUFS][3][kMaxUnits];
+  // The tile's results pass through LDS on their way out, kOutRows rows of
+  // channels at a time.
+  constexpr int kRowFloats = BN * S + 4;
+  constexpr int kLds0 = BUFS * 3 * kMaxUnits;
+  constexpr int kOutRows = UP ? 16 : kLds0 * 4 / kRowFloats >= BM ? BM
+                                 : kLds0 * 4 / kRowFloats >= 64   ? 64
+                                                                  : 32;
+  constexpr int kLds1 = (kOutRows * kRowFloats + 3) / 4;
+  constexpr int kLds = kLds0 > kLds1 ? kLds0 : kLds1;
+  static_assert(!FUSED || 3 * BM / 8 * BN <= kLds, "the second operand's LDS");
+  __shared__ uintx4 xs[kLds];
 
-  // Work-group to tile: consecutive tiles stay on one XCD, the
-  // positions of a row block where the weights are the larger operand, the
-  // row blocks of a position tile where the input is, so that the XCDs'
-  // caches do not all hold the larger one.
+  // Work-group to tile: consecutive tiles stay on one XCD, the positions of a
+  // row block where the weights are the larger operand, the row blocks of a
+  // position tile where the input is, so that the XCDs' caches do not all
+  // hold the larger one.
   const int tiles_n = (p.positions + BN - 1) / BN, tiles_m = (p.cout + BM - 1) / BM;
   int tile = XcdTile(blockIdx.x, gridDim.x), tile_n, tile_m;
   if (p.rows_first) {
@@ -131,9 +175,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
     tile /= tiles_m;
   }
   const int split = tile % p.splits;
-  const int rest = tile / p.splits;  // batch x phases + phase
-  const int phase = rest % p.phases;
-  const int batch = rest / p.phases;
+  const int batch = tile / p.splits;
   const int chunks = (p.cin + kChunk - 1) / kChunk;
   const int c_begin = split * p.split_chunks;
   const int c_end = min(chunks, c_begin + p.split_chunks);
@@ -142,28 +184,33 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
   const int co0 = tile_m * BM;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int row = (wave / WN) * 32;       // first output channel of the wave
-  const int col = (wave % WN) * 32 * NT;  // first position of the wave
-  const int half = lane >> 5;             // K half of the lane's operands
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int phase = UP ? wave : 0;
+  const int rest = UP ? wave : batch;               // the weights' lead
+  const int row = UP ? 0 : (wave / WN) * 32;        // first output channel of the wave
+  const int col = (wave % WN) * 32 * NT;            // first position of the wave
+  const int half = lane >> 5;                       // K half of the lane's operands
   const int l32 = lane & 31;
   const int dilation = TAPS == 1 ? 0 : p.dilation;
   const int width = TAPS <= 2 ? kMaxWidth : BN + (TAPS - 1) * dilation;
   const int units = kChunk / 8 * width;
+  // The window's first column is the first phase's, the least of them.
+  const int lo = p.first[0];
+  const int shift = UP ? p.first[phase] - lo : 0;
 
-  // Unit u = tid + 256 q of a chunk's window: channels 8 (u / width) .. + 7
+  // Unit u = tid + q kT of a chunk's window: channels 8 (u / width) .. + 7
   // at window column u % width.
   int at[kSlots], group[kSlots];  // first input position, 8-channel group
   unsigned inside[kSlots];        // bit i: channel i of the unit is a value
 #pragma unroll
   for (int q = 0; q < kSlots; ++q) {
-    const int u = min(tid + q * kThreads, units - 1);
+    const int u = min(tid + q * kT, units - 1);
     group[q] = u / width;
     const int m = m0 + u % width;
     if (VIEW) {
-      at[q] = m * p.view_stride + p.first[phase];
+      at[q] = m * p.view_stride + lo;
     } else {
-      const int t = m + p.first[phase];
+      const int t = m + lo;
       inside[q] = t >= 0 && t < p.len_in ? 0xFFU : 0U;
       at[q] = min(max(t, 0), p.len_in - 1);
     }
@@ -172,7 +219,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
   auto fetch = [&](int chunk) {
 #pragma unroll
     for (int q = 0; q < kSlots; ++q) {
-      if (wave * 64 + q * kThreads >= units)
+      if (wave * 64 + q * kT >= units)
         break;
       const int j = chunk * kChunk + 8 * group[q];
       if (VIEW) {
@@ -209,8 +256,8 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
   auto stash = [&](int chunk, int buf) {
 #pragma unroll
     for (int q = 0; q < kSlots; ++q) {
-      const int u = tid + q * kThreads;
-      if (wave * 64 + q * kThreads >= units)
+      const int u = tid + q * kT;
+      if (wave * 64 + q * kT >= units)
         break;
       const int j = chunk * kChunk + 8 * group[q];
       if (p.alpha_in != nullptr) {
@@ -235,7 +282,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
       if (u < units) {
 #pragma unroll
         for (int s = 0; s < 3; ++s)
-          xs[buf][s][u] = part[s];
+          xs[(buf * 3 + s) * kMaxUnits + u] = part[s];
       }
     }
   };
@@ -269,7 +316,7 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
     __syncthreads();
     if (BUFS > 1 && chunk + 1 < c_end)
       fetch(chunk + 1);
-    const uintx4* base = &xs[buf][0][half * width + col + l32];
+    const uintx4* base = xs + buf * 3 * kMaxUnits + half * width + col + l32 + shift;
     // Block i of a chunk: column block i % NT of step i / NT.
     auto read = [&](int i, uintx4* v) {
       const int step = i / NT;
@@ -287,93 +334,193 @@ __global__ __launch_bounds__(kThreads, 2) void ConvKernel(ConvParams p) {
         read(i + 1, b[(i + 1) & 1]);
       // Keeps the next block's reads ahead of this block's products.
       __builtin_amdgcn_sched_barrier(0);
-      const uintx4* aa = a[step % kAhead];
-      const uintx4* bb = b[i & 1];
-      low[t] = MfmaBf16(aa[0], bb[2], low[t]);
-      main[t] = MfmaBf16(aa[0], bb[0], main[t]);
-      low[t] = MfmaBf16(aa[2], bb[0], low[t]);
-      low[t] = MfmaBf16(aa[1], bb[1], low[t]);
-      low[t] = MfmaBf16(aa[0], bb[1], low[t]);
-      low[t] = MfmaBf16(aa[1], bb[0], low[t]);
+      Products(a[step % kAhead], b[i & 1], main[t], low[t]);
       __builtin_amdgcn_sched_barrier(0);
       if (t == NT - 1)
         load(a[step % kAhead]);
     }
   }
 
-  // Element r of the accumulators: output channel row + 8 (r / 4) +
-  // 4 half + r % 4, position col + 32 t + l32.
+  // Element r of the accumulators: output channel row + 8 (r / 4) + 4 half +
+  // r % 4, position col + 32 t + l32.
   const float* bias = p.bias != nullptr ? p.bias + batch * p.b_batch : nullptr;
-  float* y = p.y != nullptr ? p.y + batch * p.y_batch : nullptr;
-  float* y_act = p.y_act != nullptr ? p.y_act + batch * p.y_batch : nullptr;
-  const float* prior_of = p.residual != nullptr ? p.residual + batch * p.y_batch : nullptr;
-  const int co1 = co0 + row + 4 * half;
-  const int first = m0 + col + l32;
-  if (p.splits > 1) {
-    // partial[rest][split][co][m]
+  if (!FUSED && p.splits > 1) {
+    // partial[batch or phase][split][co][m]
     float* part = p.partial + (static_cast<size_t>(rest) * p.splits + split) * p.cout * p.positions;
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-      const int m = first + 32 * t;
+      const int m = m0 + col + 32 * t + l32;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const int co = co1 + 8 * (r >> 2) + (r & 3);
+        const int co = co0 + row + 8 * (r >> 2) + 4 * half + (r & 3);
         if (m < p.positions && co < p.cout)
           part[static_cast<size_t>(co) * p.positions + m] = Join(main[t][r], low[t][r]);
       }
     }
     return;
   }
-  // Four channels at a time. Every load of a group (bias, the residual, the
-  // Snake alphas) is issued before the previous group's stores: the stores may
-  // alias them as far as the compiler knows, so loads left between them would
-  // each wait out a memory round trip.
-  struct Group {
-    float bias[4], alpha[4], residual[NT][4];
+
+  if (FUSED) {
+    // The second convolution: 8 channels of a position are the 4 + 4 of a
+    // lane pair.
+    const uintx4* w2 = reinterpret_cast<const uintx4*>(p.w2) +
+                       static_cast<size_t>(half) * p.w_rows + min(row + l32, p.w_rows - 1);
+    auto load2 = [&](int step, uintx4* v) {
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+        v[s] = w2[(static_cast<size_t>(step) * 6 + 2 * s) * p.w_rows];
+    };
+    load2(0, a[0]);
+    __syncthreads();
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      float bias4[4], alpha4[4], inverse4[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int co = min(row + 8 * g + 4 * half + r, p.cout - 1);
+        bias4[r] = bias[co];
+        alpha4[r] = p.alpha_mid[co];
+        inverse4[r] = SnakeInverse(alpha4[r]);
+      }
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        float v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          v[r] = Snake(Join(main[t][4 * g + r], low[t][4 * g + r]) + bias4[r], alpha4[r],
+                       inverse4[r]);
+          v[r] = row + 8 * g + 4 * half + r < p.cout ? v[r] : 0.0F;
+        }
+        floatx2 rest0{v[0], v[1]}, rest1{v[2], v[3]};
+        auto* to = reinterpret_cast<uintx2*>(xs + (row / 8 + g) * BN + col + 32 * t + l32) + half;
+#pragma unroll
+        for (int s = 0; s < 3; ++s) {
+          const uintx2 pairs{RoundPair(rest0), RoundPair(rest1)};
+          to[s * 2 * (BM / 8 * BN)] = pairs;
+          rest0 = Rest(rest0, pairs[0]);
+          rest1 = Rest(rest1, pairs[1]);
+        }
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      main[t] = low[t] = floatx16{};
+    const uintx4* base = xs + half * BN + col + l32;
+#pragma unroll
+    for (int step = 0; step < BM / 16; ++step) {
+      if (step + 1 < BM / 16)
+        load2(step + 1, a[(step + 1) & 1]);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) {
+        uintx4 v[3];
+#pragma unroll
+        for (int s = 0; s < 3; ++s)
+          v[s] = base[s * (BM / 8 * BN) + 2 * step * BN + 32 * t];
+        Products(a[step & 1], v, main[t], low[t]);
+      }
+    }
+    bias = p.bias2;
+  }
+
+  // Out through LDS, as rows of positions, then in a loop over 16-byte runs:
+  // the residual loads and the stores are wide, and the code that every
+  // work-group runs once, and has to fetch, is short (straight from the
+  // accumulators it was most of the kernel). Four runs at a time, the next
+  // four's loads issued before these four's stores, which may alias them as
+  // far as the compiler knows.
+  float* y = p.y != nullptr ? p.y + batch * p.y_batch : nullptr;
+  float* y_act = p.y_act != nullptr ? p.y_act + batch * p.y_batch : nullptr;
+  const float* residual = p.residual != nullptr ? p.residual + batch * p.y_batch : nullptr;
+  constexpr int kRuns = BN * S / 4;      // per row
+  constexpr int kStride = kT / kRuns;    // rows between a thread's runs
+  constexpr int kPer = kOutRows / kStride / 4;
+  static_assert(kT % kRuns == 0 && kOutRows % (4 * kStride) == 0, "runs");
+  const int length = p.positions * S;
+  const int at0 = m0 * S + tid % kRuns * 4;  // the thread's first output position
+  const int n = min(length - at0, 4);
+  struct Runs {
+    float bias[4], alpha[4];
+    floatx4 residual[4];
   };
-  auto gather = [&](int g) {
-    Group v;
+  auto gather = [&](int first) {
+    Runs v;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int co = min(co1 + 8 * g + r, p.cout - 1);
-      v.bias[r] = bias != nullptr ? bias[co] : 0.0F;
-      v.alpha[r] = y_act != nullptr && p.out_act == kActSnake ? p.alpha_out[co] : 0.0F;
-#pragma unroll
-      for (int t = 0; t < NT; ++t)
-        v.residual[t][r] =
-            prior_of != nullptr
-                ? prior_of[static_cast<size_t>(co) * p.len_out +
-                           static_cast<size_t>(min(first + 32 * t, p.positions - 1)) * p.out_stride +
-                           phase]
-                : 0.0F;
+    for (int i = 0; i < 4; ++i) {
+      const int co = min(co0 + first + i * kStride, p.cout - 1);
+      v.bias[i] = bias != nullptr ? bias[co] : 0.0F;
+      v.alpha[i] = y_act != nullptr && p.out_act == kActSnake ? p.alpha_out[co] : 0.0F;
+      v.residual[i] = floatx4{0.0F, 0.0F, 0.0F, 0.0F};
+      if (residual != nullptr && n > 0) {
+        const float* from = residual + static_cast<size_t>(co) * p.len_out + at0;
+        if (n == 4)
+          v.residual[i] = *reinterpret_cast<const Unaligned4*>(from);
+        else
+          for (int e = 0; e < n; ++e)
+            v.residual[i][e] = from[e];
+      }
     }
     return v;
   };
-  Group next = gather(0);
+  float* out = reinterpret_cast<float*>(xs);
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const Group cur = next;
-    if (g < 3)
-      next = gather(g + 1);
-    __builtin_amdgcn_sched_barrier(0);
+  for (int r0 = 0; r0 < BM; r0 += kOutRows) {
+    const int mine = r0 + tid / kRuns;
+    Runs next = gather(mine);
+    __syncthreads();
+    if (UP) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int co = co1 + 8 * g + r;
-      const float inverse = SnakeInverse(cur.alpha[r]);
+      for (int t = 0; t < NT; ++t)
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int m = first + 32 * t;
-        if (m < p.positions && co < p.cout) {
-          const size_t to = static_cast<size_t>(co) * p.len_out +
-                            static_cast<size_t>(m) * p.out_stride + phase;
-          float v = Join(main[t][4 * g + r], low[t][4 * g + r]) + cur.bias[r];
+        for (int r = 0; r < 8; ++r)
+          out[(8 * (r >> 2) + 4 * half + (r & 3)) * kRowFloats + (32 * t + l32) * S + phase] =
+              Join(main[t][r0 / 2 + r], low[t][r0 / 2 + r]);
+    } else if (row >= r0 && row < r0 + kOutRows) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          out[(row - r0 + 8 * (r >> 2) + 4 * half + (r & 3)) * kRowFloats + col + 32 * t + l32] =
+              Join(main[t][r], low[t][r]);
+    }
+    __syncthreads();
+#pragma unroll 1
+    for (int q = 0; q < kPer; ++q) {
+      const Runs cur = next;
+      if (q + 1 < kPer)
+        next = gather(mine + 4 * (q + 1) * kStride);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int local = mine + (4 * q + i) * kStride;
+        if (co0 + local >= p.cout || n <= 0)
+          continue;
+        floatx4 v = *reinterpret_cast<const floatx4*>(out + (local - r0) * kRowFloats +
+                                                      tid % kRuns * 4);
+        const size_t to = static_cast<size_t>(co0 + local) * p.len_out + at0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          v[e] += cur.bias[i];
           if (p.pre_act == kActGelu)
-            v = Gelu(v);
-          v += cur.residual[t][r];
-          if (y != nullptr)
-            y[to] = v;
-          if (y_act != nullptr)
-            y_act[to] = p.out_act == kActElu ? Elu(v) : Snake(v, cur.alpha[r], inverse);
+            v[e] = Gelu(v[e]);
+          v[e] += cur.residual[i][e];
+        }
+        if (y != nullptr) {
+          if (n == 4)
+            *reinterpret_cast<Unaligned4*>(y + to) = v;
+          else
+            for (int e = 0; e < n; ++e)
+              y[to + e] = v[e];
+        }
+        if (y_act != nullptr) {
+          const float inverse = SnakeInverse(cur.alpha[i]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[e] = p.out_act == kActElu ? Elu(v[e]) : Snake(v[e], cur.alpha[i], inverse);
+          if (n == 4)
+            *reinterpret_cast<Unaligned4*>(y_act + to) = v;
+          else
+            for (int e = 0; e < n; ++e)
+              y_act[to + e] = v[e];
         }
       }
     }
@@ -433,7 +580,7 @@ __global__ __launch_bounds__(kThreads) void SplitReduceKernel(ConvParams p) {
     float* y = p.y != nullptr ? p.y + batch * p.y_batch : nullptr;
     float* y_act = p.y_act != nullptr ? p.y_act + batch * p.y_batch : nullptr;
     const float* residual = p.residual != nullptr ? p.residual + batch * p.y_batch : nullptr;
-    const size_t t = static_cast<size_t>(m) * p.out_stride + phase;
+    const size_t t = static_cast<size_t>(m) * p.phases + phase;
     Finish(p, bias, residual, y, y_act, co, static_cast<size_t>(co) * p.len_out + t, v);
   }
 }
@@ -489,65 +636,97 @@ __global__ __launch_bounds__(kThreads) void RvqKernel(RvqParams p) {
   }
 }
 
-template <int WM, int WN, int NT, int TAPS, int BUFS, bool VIEW>
+template <int WM, int WN, int NT, int TAPS, int BUFS, ConvKind KIND>
 void DispatchTile(const ConvParams& p, hipStream_t stream) {
-  constexpr int BM = 32 * WM, BN = 32 * WN * NT;
+  constexpr int BM = KIND == kUp ? 32 : 32 * WM, BN = 32 * WN * NT;
   const int64_t grid = static_cast<int64_t>((p.positions + BN - 1) / BN) *
-                       ((p.cout + BM - 1) / BM) * p.phases * p.batches * p.splits;
+                       ((p.cout + BM - 1) / BM) * p.batches * p.splits;
   Require(grid < (int64_t{1} << 31), "conv: too many tiles");
-  Dispatch(ConvKernel<WM, WN, NT, TAPS, BUFS, VIEW>, dim3(static_cast<unsigned>(grid)),
-           dim3(kThreads), 0, stream, true, p.splits == 1, p);
+  Dispatch(ConvKernel<WM, WN, NT, TAPS, BUFS, KIND>, dim3(static_cast<unsigned>(grid)),
+           dim3(64 * WM * WN), 0, stream, true, p.splits == 1, p);
+}
+
+// Splits the input channels of a convolution whose tiles number under 256
+// until about 512 work-groups run, if there is a workspace.
+void ChooseSplits(ConvParams* p, int64_t tiles, int chunk) {
+  const int chunks = (p->cin + chunk - 1) / chunk;
+  p->splits = 1;
+  p->split_chunks = chunks;
+  if (p->partial == nullptr || tiles >= 256 || chunks < 4)
+    return;
+  int64_t want = std::min<int64_t>((512 + tiles - 1) / tiles, chunks / 2);
+  const int64_t outputs = static_cast<int64_t>(p->cout) * p->positions * p->phases * p->batches;
+  want = std::min<int64_t>(want, p->partial_capacity / std::max<int64_t>(outputs, 1));
+  want = std::min<int64_t>(want, 65535 / (static_cast<int64_t>(p->phases) * p->batches));
+  if (want >= 2) {
+    p->split_chunks = static_cast<int>((chunks + want - 1) / want);
+    p->splits = (chunks + p->split_chunks - 1) / p->split_chunks;
+  }
+}
+
+void Reduce(const ConvParams& p, hipStream_t stream) {
+  if (p.splits == 1)
+    return;
+  const size_t total = static_cast<size_t>(p.cout) * p.positions * p.phases * p.batches;
+  const int blocks = static_cast<int>(std::min<size_t>((total + kThreads - 1) / kThreads, 16384));
+  Dispatch(SplitReduceKernel, dim3(blocks), dim3(kThreads), 0, stream, false, true, p);
+}
+
+int64_t Tiles(const ConvParams& p, int bm, int bn) {
+  return static_cast<int64_t>((p.positions + bn - 1) / bn) * ((p.cout + bm - 1) / bm) * p.batches;
 }
 
 // The tile: all output channels of a narrow layer (32 x 256 when the input is
 // one chunk, so that two work-groups' windows fit a CU's LDS, else 32 x 128;
 // 64 x 128), else 128 x 128 where that gives every CU a work-group, else
 // 128 x 64.
-//
-// With a split-K workspace, a convolution whose tiles number under 256
-// instead splits its input channels until about 512 work-groups run, and a
-// reduction kernel finishes it.
-template <int TAPS, bool VIEW>
+template <int TAPS, ConvKind KIND>
 void DispatchTaps(const ConvParams& params, hipStream_t stream) {
   ConvParams p = params;
-  const auto groups = [&](int bm, int bn) {
-    return static_cast<int64_t>((p.positions + bn - 1) / bn) * ((p.cout + bm - 1) / bm) *
-           p.phases * p.batches;
-  };
-  const int64_t inputs = static_cast<int64_t>(VIEW ? p.channels : p.cin) * p.len_in * p.batches;
-  p.rows_first = 2 * inputs > int64_t{3} * p.taps * p.cin * p.cout * p.phases * p.batches;
-  const bool wide = p.cout > 64 && groups(128, 128) >= 256;
+  const bool wide = p.cout > 64 && Tiles(p, 128, 128) >= 256;
   const bool one = p.cin <= 32;
   const int columns = p.cout <= 32 ? (one ? 256 : 128) : p.cout <= 64 || wide ? 128 : 64;
-  const int64_t tiles = groups(p.cout <= 32 ? 32 : p.cout <= 64 ? 64 : 128, columns);
-  const int chunk = TileChunk(TAPS, columns), chunks = (p.cin + chunk - 1) / chunk;
-  p.splits = 1;
-  p.split_chunks = chunks;
-  if (p.partial != nullptr && tiles < 256 && chunks >= 4) {
-    int64_t want = std::min<int64_t>((512 + tiles - 1) / tiles, chunks / 2);
-    const int64_t outputs = static_cast<int64_t>(p.cout) * p.positions * p.phases * p.batches;
-    want = std::min<int64_t>(want, p.partial_capacity / std::max<int64_t>(outputs, 1));
-    want = std::min<int64_t>(want, 65535 / (static_cast<int64_t>(p.phases) * p.batches));
-    if (want >= 2) {
-      p.split_chunks = static_cast<int>((chunks + want - 1) / want);
-      p.splits = (chunks + p.split_chunks - 1) / p.split_chunks;
-    }
-  }
+  ChooseSplits(&p, Tiles(p, p.cout <= 32 ? 32 : p.cout <= 64 ? 64 : 128, columns),
+               TileChunk(TAPS, columns));
   if (p.cout <= 32 && one)
-    DispatchTile<1, 4, 2, TAPS, 1, VIEW>(p, stream);
+    DispatchTile<1, 4, 2, TAPS, 1, KIND>(p, stream);
   else if (p.cout <= 32)
-    DispatchTile<1, 4, 1, TAPS, 2, VIEW>(p, stream);
+    DispatchTile<1, 4, 1, TAPS, 2, KIND>(p, stream);
   else if (p.cout <= 64)
-    DispatchTile<2, 2, 2, TAPS, 2, VIEW>(p, stream);
+    DispatchTile<2, 2, 2, TAPS, 2, KIND>(p, stream);
   else if (wide)
-    DispatchTile<4, 1, 4, TAPS, 2, VIEW>(p, stream);
+    DispatchTile<4, 1, 4, TAPS, 2, KIND>(p, stream);
   else
-    DispatchTile<4, 1, 2, TAPS, 2, VIEW>(p, stream);
-  if (p.splits > 1) {
-    const size_t total = static_cast<size_t>(p.cout) * p.positions * p.phases * p.batches;
-    const int blocks = static_cast<int>(std::min<size_t>((total + kThreads - 1) / kThreads, 16384));
-    Dispatch(SplitReduceKernel, dim3(blocks), dim3(kThreads), 0, stream, false, true, p);
+    DispatchTile<4, 1, 2, TAPS, 2, KIND>(p, stream);
+  Reduce(p, stream);
+}
+
+// A residual unit of up to 128 channels in one launch.
+void DispatchFused(const ConvParams& params, hipStream_t stream) {
+  ConvParams p = params;
+  ChooseSplits(&p, 256, 32);
+  if (p.cout <= 32)
+    DispatchTile<1, 4, 2, 7, 1, kFused>(p, stream);
+  else if (p.cout <= 64)
+    DispatchTile<2, 2, 2, 7, 2, kFused>(p, stream);
+  else
+    DispatchTile<4, 1, 2, 7, 2, kFused>(p, stream);
+}
+
+// A transposed convolution: a wave per phase.
+void DispatchUp(const ConvParams& params, hipStream_t stream) {
+  ConvParams p = params;
+  ChooseSplits(&p, Tiles(p, 32, 64), 32);
+  switch (p.phases) {
+    case 2: DispatchTile<2, 1, 2, 2, 2, kUp>(p, stream); break;
+    case 3: DispatchTile<3, 1, 2, 2, 2, kUp>(p, stream); break;
+    case 4: DispatchTile<4, 1, 2, 2, 2, kUp>(p, stream); break;
+    case 5: DispatchTile<5, 1, 2, 2, 2, kUp>(p, stream); break;
+    case 6: DispatchTile<6, 1, 2, 2, 2, kUp>(p, stream); break;
+    case 7: DispatchTile<7, 1, 2, 2, 2, kUp>(p, stream); break;
+    default: DispatchTile<8, 1, 2, 2, 2, kUp>(p, stream); break;
   }
+  Reduce(p, stream);
 }
 
 }  // namespace
@@ -590,8 +769,11 @@ void LaunchConv(const ConvParams& params, hipStream_t stream) {
           "conv: empty shape");
   Require(p.taps == 1 || p.taps == 2 || p.taps == 7, "conv: 1, 2 or 7 taps");
   Require(p.phases >= 1 && p.phases <= kConvMaxPhases, "conv: 1 to 8 phases");
-  Require(p.out_stride >= p.phases, "conv: phases overlap in the output");
-  Require(static_cast<int64_t>(p.positions - 1) * p.out_stride + p.phases - 1 < p.len_out,
+  Require(p.phases == 1 || (p.taps == 2 && p.batches == 1), "conv: phases have two taps");
+  for (int i = 1; i < p.phases; ++i)
+    Require(p.first[i] - p.first[0] == 0 || p.first[i] - p.first[0] == 1,
+            "conv: the phases' windows differ by one position at most");
+  Require(static_cast<int64_t>(p.positions) * p.phases <= p.len_out,
           "conv: output positions past the output length");
   Require(p.taps == 1 || (p.dilation >= 1 &&
                           (p.taps - 1) * static_cast<int64_t>(p.dilation) <=
@@ -604,13 +786,21 @@ void LaunchConv(const ConvParams& params, hipStream_t stream) {
                 (p.positions + int64_t{256}) * p.view_stride + p.view_kernel <
                     (std::int64_t{1} << 31),
             "conv: bad view");
-    DispatchTaps<1, true>(p, stream);
+    DispatchTaps<1, kView>(p, stream);
+  } else if (p.w2 != nullptr) {
+    Require(p.taps == 7 && p.batches == 1 && p.cin == p.cout && p.cout <= kConvFusedChannels &&
+                p.bias != nullptr && p.bias2 != nullptr && p.alpha_mid != nullptr &&
+                p.pre_act == kActNone && p.x != p.y && p.x != p.y_act,
+            "conv: bad residual unit");
+    DispatchFused(p, stream);
+  } else if (p.phases > 1) {
+    DispatchUp(p, stream);
   } else if (p.taps == 1) {
-    DispatchTaps<1, false>(p, stream);
+    DispatchTaps<1, kPlain>(p, stream);
   } else if (p.taps == 2) {
-    DispatchTaps<2, false>(p, stream);
+    DispatchTaps<2, kPlain>(p, stream);
   } else {
-    DispatchTaps<7, false>(p, stream);
+    DispatchTaps<7, kPlain>(p, stream);
   }
 }
 

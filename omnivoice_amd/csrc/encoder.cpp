@@ -166,6 +166,8 @@ class EncoderEngine {
   void RunConv7(const Conv7& c, const float* x, int length, float* y, float* y_act,
                 const float* alpha_out, bool accumulate, hipStream_t stream, Profiler* prof,
                 const char* name);
+  void RunUnit(const Unit& unit, const float* x, int length, float* y_act,
+               const float* alpha_out, hipStream_t stream, Profiler* prof);
 
   ovc_encoder_config cfg_;
   int W_ = 0, H_ = 0;
@@ -551,7 +553,6 @@ void EncoderEngine::RunGemm(const Gemm& g, hipStream_t stream, Profiler* prof,
   p.taps = 1;
   p.phases = 1;
   p.positions = g.positions;
-  p.out_stride = 1;
   if (g.len_in > 0) {
     p.view_kernel = g.d->kernel;
     p.view_stride = g.stride;
@@ -593,7 +594,6 @@ void EncoderEngine::RunConv7(const Conv7& c, const float* x, int length, float* 
   p.taps = 7;
   p.phases = 1;
   p.positions = length;
-  p.out_stride = 1;
   p.residual = accumulate ? y : nullptr;
   p.partial = partial_.get();
   p.partial_capacity = kPartialFloats;
@@ -605,6 +605,35 @@ void EncoderEngine::RunConv7(const Conv7& c, const float* x, int length, float* 
   auto launch = [&] { LaunchConv(p, stream); };
   if (prof != nullptr)
     prof->Run(name, flops, bytes, launch);
+  else
+    launch();
+}
+
+// A whole residual unit: x_ += conv2(snake(conv1(x))), y_act its Snake.
+void EncoderEngine::RunUnit(const Unit& unit, const float* x, int length, float* y_act,
+                            const float* alpha_out, hipStream_t stream, Profiler* prof) {
+  const Conv7& c = unit.conv1;
+  ConvParams p{};
+  p.x = x;
+  p.w = c.w.get();
+  p.bias = c.b.get();
+  p.w2 = unit.conv2.w.get();
+  p.bias2 = unit.conv2.b.get();
+  p.alpha_mid = unit.alpha2.get();
+  p.residual = p.y = x_.get();
+  p.y_act = y_act;
+  p.alpha_out = alpha_out;
+  p.cin = p.cout = c.out;
+  p.len_in = p.len_out = p.positions = length;
+  p.taps = 7;
+  p.phases = 1;
+  p.dilation = c.dilation;
+  p.first[0] = -3 * c.dilation;
+  const double flops = 2.0 * c.out * static_cast<double>(length) * c.out * 8;
+  const double bytes = 16.0 * length * c.out + 32.0 * c.out * c.out;
+  auto launch = [&] { LaunchConv(p, stream); };
+  if (prof != nullptr)
+    prof->Run("enc_dac_res_unit", flops, bytes, launch);
   else
     launch();
 }
@@ -690,7 +719,6 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
     p.taps = 1;
     p.phases = 1;
     p.positions = T;
-    p.out_stride = 1;
     p.pre_act = kActGelu;
     p.batches = G;
     p.partial = partial_.get();
@@ -812,6 +840,12 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
     const Block& blk = *blocks_[bi];
     for (int u = 0; u < 3; ++u) {
       const Unit& unit = blk.units[u];
+      const float* next_alpha = u < 2 ? blk.units[u + 1].alpha1.get() : blk.alpha.get();
+      if (blk.channels <= kConvFusedChannels) {
+        RunUnit(unit, xa, cur, ya, next_alpha, stream, prof);
+        std::swap(xa, ya);
+        continue;
+      }
       RunConv7(unit.conv1, xa, cur, nullptr, ya, unit.alpha2.get(), false, stream,
                prof, "enc_dac_res_conv7");
       Gemm g;
@@ -820,7 +854,7 @@ void EncoderEngine::Enqueue(const float* samples, const Plan& plan, std::int32_t
       g.y = x_.get();
       g.y_act = xa;
       g.out_act = kActSnake;
-      g.alpha_out = u < 2 ? blk.units[u + 1].alpha1.get() : blk.alpha.get();
+      g.alpha_out = next_alpha;
       g.positions = cur;
       g.accumulate = true;
       RunGemm(g, stream, prof, "enc_dac_res_conv1");

@@ -95,6 +95,41 @@ def test_conv1d_tile_edges(cin, cout, length, kernel, dilation):
     assert (np.abs(y.cpu().numpy() - want) <= (cin * kernel / 8 + 8) * 2.0 ** -24 * size).all()
 
 
+@pytest.mark.parametrize("cin,cout,length,stride", [
+    (32, 31, 1, 1), (33, 33, 63, 2), (31, 64, 65, 3), (64, 96, 64, 4), (65, 40, 129, 5),
+    (40, 32, 33, 6), (16, 65, 100, 7), (128, 20, 66, 8)])
+def test_conv_transpose1d_tile_edges(cin, cout, length, stride):
+    """Every stride at the edges of the tiles against 64 bits, with the bound of the test above
+    (two taps reach each output)."""
+    rng = np.random.default_rng(cin + cout + length)
+    x = rng.standard_normal((cin, length)).astype(np.float32)
+    w = (rng.standard_normal((cin, cout, 2 * stride)) / math.sqrt(2 * cin)).astype(np.float32)
+    b = rng.standard_normal(cout).astype(np.float32)
+    y = dev(np.zeros((cout, length * stride)))
+    ov.op_conv_transpose1d(dev(x), w, b, y, stride)
+
+    def run(x, w, b):
+        full = np.zeros((cout, (length + 2) * stride))
+        for k in range(2 * stride):
+            full[:, k:k + (length - 1) * stride + 1:stride] += w[:, :, k].T @ x
+        pad = (stride + 1) // 2
+        return full[:, pad:pad + length * stride] + b[:, None]
+    x, w, b = (v.astype(np.float64) for v in (x, w, b))
+    size = run(np.abs(x), np.abs(w), np.abs(b))
+    bound = (2 * cin / 8 + 8) * 2.0 ** -24 * size
+    assert (np.abs(y.cpu().numpy() - run(x, w, b)) <= bound).all()
+
+
+@pytest.mark.parametrize("channels,frames", [(32, 5), (64, 11), (128, 23), (192, 43), (256, 3)])
+def test_fused_residual_units_match_oracle(channels, frames):
+    """Decoders whose blocks' units run fused at every tile (16 to 128 channels, ragged ones
+    too), next to 256 channels that do not."""
+    cfg = dict(TINY, channels=channels * 2, ratios=[5, 2])
+    codes = np.random.default_rng(frames).integers(0, 16, size=(3, frames)).astype(np.int32)
+    close(ov.Codec.synthetic(cfg, 31).decode(codes), oracle.Codec(cfg, 31).decode(codes),
+          rtol=2e-4)
+
+
 def test_conv1d_keeps_infinities():
     """An infinite input makes its outputs infinite, not NaN; NaN stays where it reaches."""
     x = np.ones((32, 200), dtype=np.float32)

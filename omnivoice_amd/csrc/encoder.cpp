@@ -190,7 +190,7 @@ class EncoderEngine {
   std::vector<std::unique_ptr<Stage>> stages_;
   DeviceBuffer<RvqStage> stage_list_;
   // work buffers
-  DeviceBuffer<float> samples_, wave_, fa_, fb_, tmp_, h_, qkv_, ctx_, ff_;
+  DeviceBuffer<float> samples_, wave_, fa_, fb_, turned_, tmp_, h_, qkv_, ctx_, ff_;
   DeviceBuffer<double> sum_;
   DeviceBuffer<std::uint16_t> heads_;  // the attention's operands
   // Split-K workspace of the thin GEMMs (HuBERT at short lengths, the
@@ -916,19 +916,21 @@ void EncoderEngine::Encode(const float* samples, int64_t length, std::int32_t* c
   Check(hipMemcpyAsync(codes, codes_.get(), sizeof(std::int32_t) * cfg_.codebooks * F,
                        hipMemcpyDeviceToHost, stream_),
         "download codes");
-  // Optional intermediate outputs, frame-major: [frames][channels].
+  // Optional intermediate outputs, frame-major: [frames][channels], turned on
+  // the device (a host loop over the strided columns took longer than a third
+  // of the encode: 5 of 13.5 ms at 523 frames).
   auto download = [&](const float* dev, int64_t rows, float* out) {
     if (out == nullptr)
       return;
-    std::vector<float> host(static_cast<std::size_t>(rows * F));
-    Check(hipMemcpyAsync(host.data(), dev, sizeof(float) * rows * F, hipMemcpyDeviceToHost,
-                         stream_),
+    float* turned = turned_.get();
+    LaunchTranspose(dev, turned, static_cast<int>(rows), static_cast<int>(F), stream_);
+    Check(hipMemcpyAsync(out, turned, sizeof(float) * rows * F, hipMemcpyDeviceToHost, stream_),
           "download");
-    Check(hipStreamSynchronize(stream_), "encode");
-    for (int64_t r = 0; r < rows; ++r)
-      for (int64_t f = 0; f < F; ++f)
-        out[f * rows + r] = host[static_cast<std::size_t>(r * F + f)];
   };
+  if (semantic != nullptr || acoustic != nullptr || embeddings != nullptr) {
+    if (turned_.size() < static_cast<std::size_t>(std::max(W, H) * F))
+      turned_.Reserve(static_cast<std::size_t>(std::max(W, H) * F));
+  }
   download(sem_.get(), W, semantic);
   download(joint_.get(), lat, acoustic);
   download(emb_.get(), H, embeddings);

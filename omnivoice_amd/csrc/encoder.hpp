@@ -22,6 +22,9 @@ struct ResampleParams {
 };
 void LaunchResample(const ResampleParams& p, hipStream_t stream);
 
+// y [cols][rows] = x [rows][cols] transposed.
+void LaunchTranspose(const float* x, float* y, int rows, int cols, hipStream_t stream);
+
 // GroupNorm with one group per channel (statistics over the row), affine,
 // then GELU, in place: x [channels][length].
 void LaunchGroupNormGelu(float* x, const float* w, const float* b, int channels, int length,

@@ -49,6 +49,21 @@ __global__ __launch_bounds__(kThreads) void ResampleKernel(ResampleParams p) {
   }
 }
 
+// 32 x 32 tiles through LDS, both sides in whole 128-byte runs.
+__global__ __launch_bounds__(kThreads) void TransposeKernel(const float* x, float* y, int rows,
+                                                            int cols) {
+  __shared__ float tile[32][33];
+  const int c0 = blockIdx.x * 32, r0 = blockIdx.y * 32;
+  const int i = threadIdx.x % 32;
+  for (int j = threadIdx.x / 32; j < 32; j += kThreads / 32)
+    if (r0 + j < rows && c0 + i < cols)
+      tile[j][i] = x[static_cast<size_t>(r0 + j) * cols + c0 + i];
+  __syncthreads();
+  for (int j = threadIdx.x / 32; j < 32; j += kThreads / 32)
+    if (c0 + j < cols && r0 + i < rows)
+      y[static_cast<size_t>(c0 + j) * rows + r0 + i] = tile[i][j];
+}
+
 // Sum of one double per thread over the work-group (every thread gets it).
 __device__ double BlockSum(double v, double* scratch) {
   for (int o = 32; o > 0; o >>= 1)
@@ -572,6 +587,13 @@ int Blocks(size_t work) {
 }
 
 }  // namespace
+
+void LaunchTranspose(const float* x, float* y, int rows, int cols, hipStream_t stream) {
+  Require(x && y, "transpose: null pointer");
+  Require(rows >= 1 && cols >= 1 && rows <= 32 * 65535, "transpose: bad shape");
+  Dispatch(TransposeKernel, dim3((cols + 31) / 32, (rows + 31) / 32), dim3(kThreads), 0, stream,
+           true, true, x, y, rows, cols);
+}
 
 void LaunchResample(const ResampleParams& p, hipStream_t stream) {
   Require(p.x && p.bank && p.y, "resample: null pointer");

@@ -30,7 +30,7 @@ enum ConvAct : int {
 // Float32 weights as the bf16 triples the kernel multiplies (split.hpp), in
 // units of eight input channels of one output channel; rows (output channels)
 // are padded to whole 32-row blocks, input channels to whole groups of ConvPad.
-constexpr int ConvPad(int taps) { return taps == 1 ? 64 : 32; }
+constexpr int ConvPad(int taps) { return taps == 1 ? 128 : 32; }
 struct alignas(16) ConvUnit {
   std::uint32_t pairs[4];
 };

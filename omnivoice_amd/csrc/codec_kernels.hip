@@ -70,15 +70,34 @@ __device__ __forceinline__ void Finish(const ConvParams& p, const float* bias,
 // Four floats at any 4-byte address.
 typedef float Unaligned4 __attribute__((ext_vector_type(4), aligned(4)));
 
-// The six products of a step's 32 x 32 block.
-__device__ __forceinline__ void Products(const uintx4* a, const uintx4* b, floatx16& main,
-                                         floatx16& low) {
-  low = MfmaBf16(a[0], b[2], low);
-  main = MfmaBf16(a[0], b[0], main);
-  low = MfmaBf16(a[2], b[0], low);
-  low = MfmaBf16(a[1], b[1], low);
-  low = MfmaBf16(a[0], b[1], low);
-  low = MfmaBf16(a[1], b[0], low);
+// The six products of a step's one or two 32 x 32 blocks, part by part of the
+// operand b, whose parts are read again for the next step (next(part)) as
+// soon as they are done with. A product waits some 90 cycles for the one
+// before it on the same accumulator but only 32 for the pipe, so two blocks
+// (or, for a single one, two low accumulators) are multiplied in turn; the
+// scheduling barriers keep the order, which the compiler would otherwise turn
+// back into one chain after the other. other(k) is vector work to put behind
+// product k.
+template <int N, typename Next, typename Other>
+__device__ __forceinline__ void Products(const uintx4* a, const uintx4 (*b)[3], floatx16* main,
+                                         floatx16* low, Next&& next, Other&& other) {
+  auto multiply = [&](int k, int i, int j, floatx16* sum) {
+#pragma unroll
+    for (int t = 0; t < N; ++t)
+      sum[t] = MfmaBf16(a[i], b[t][j], sum[t]);
+    other(k);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  floatx16* second = N == 1 ? low + 1 : low;
+  multiply(0, 0, 2, low);
+  next(2);
+  multiply(1, 0, 1, second);
+  multiply(2, 1, 1, low);
+  next(1);
+  multiply(3, 0, 0, main);
+  multiply(4, 1, 0, second);
+  multiply(5, 2, 0, low);
+  next(0);
 }
 
 // Work-group `id` of `count` to a tile such that each XCD (id % 8) has a run
@@ -90,7 +109,9 @@ __device__ __forceinline__ int XcdTile(int id, int count) {
 
 // Input channels per chunk of a tile (a divisor of the weights' padding): two
 // work-groups' windows fit a CU's LDS.
-constexpr int TileChunk(int taps, int columns) { return taps == 1 && columns <= 64 ? 64 : 32; }
+constexpr int TileChunk(int taps, int columns) {
+  return taps > 1 || columns > 64 ? 32 : columns == 64 ? 64 : 128;
+}
 
 // One float32 convolution as an implicit GEMM over bf16 triples (split.hpp):
 // rows are output channels, columns output positions, the sum runs over
@@ -119,12 +140,13 @@ constexpr int TileChunk(int taps, int columns) { return taps == 1 && columns <= 
 // Bound by the matrix cores (their pipes 52-60 % busy at the 1.9 GHz this
 // work draws) at 128 channels and more; at 32 and 64 by them, the activations'
 // vector work and memory alike. At a 60 s signal: the k7 convolutions of 256
-// and 512 channels 195 TFLOP/s of float32 products (87 on the float32 matrix
-// cores), a residual unit of 128 / 64 / 32 channels 379 / 278 / 301 us where
-// its two launches took 492 / 329 / 397, the transposed convolutions 230 us
+// and 512 channels 200 TFLOP/s of float32 products (87 on the float32 matrix
+// cores), a residual unit of 128 / 64 / 32 channels 400 / 273 / 300 us where
+// its two launches took 492 / 329 / 397, the transposed convolutions 204 us
 // a launch where one phase per work-group, its outputs scattered, took 295.
-// Blocks multiplied two in turn, or the fused tiles' weights seven steps
-// ahead, cost the third wave per SIMD (379 -> 441, 407 us).
+// Splitting a chunk between its predecessor's products instead of before its
+// own: one-tap layers of 768 to 3072 channels at 500 positions 22.3 -> 20.6
+// and 28.8 -> 25.0 us, the transposed convolutions 230 -> 204 us.
 enum ConvKind : int { kPlain, kView, kFused, kUp };
 
 template <int WM, int WN, int NT, int TAPS, int BUFS, ConvKind KIND>
@@ -137,19 +159,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
   constexpr int BM = UP ? 32 : 32 * WM, BN = 32 * WN * NT;
   constexpr int kChunk = TileChunk(TAPS, BN);
   constexpr int kMaxWidth = BN + (TAPS == 1 ? 0 : UP ? 2 : TAPS == 2 ? 1 : kConvMaxSpan);
-  constexpr int kMaxUnits = kChunk / 8 * kMaxWidth;
-  constexpr int kSlots = (kMaxUnits + kT - 1) / kT;
+  constexpr int kSlots = (kChunk / 8 * kMaxWidth + kT - 1) / kT;
+  constexpr int kMaxUnits = kSlots * kT;  // whole turns of the threads
   constexpr int kSubs = kChunk / 16;
   constexpr int kSteps = kSubs * TAPS;  // of 16 channels, per chunk
   // Steps the weights are loaded ahead: a narrow tile's short steps and large
   // weights need more.
-  constexpr int kAhead = NT == 4 || FUSED ? 2 : TAPS == 7 ? 7 : UP || WM == 4 ? 4 : 2;
+  constexpr int kAhead = TAPS == 7 ? 2 : BN == 32 && TAPS == 1 ? 8 : UP || WM == 4 ? 4 : 2;
   static_assert(kSteps % kAhead == 0, "weight registers");
   // The tile's results pass through LDS on their way out, kOutRows rows of
   // channels at a time.
   constexpr int kRowFloats = BN * S + 4;
   constexpr int kLds0 = BUFS * 3 * kMaxUnits;
-  constexpr int kOutRows = UP ? 16 : kLds0 * 4 / kRowFloats >= BM ? BM
+  constexpr int kOutRows = UP ? 16 : kLds0 * 4 / kRowFloats >= BM || BN == 32 ? BM
                                  : kLds0 * 4 / kRowFloats >= 64   ? 64
                                                                   : 32;
   constexpr int kLds1 = (kOutRows * kRowFloats + 3) / 4;
@@ -201,7 +223,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
   // Unit u = tid + q kT of a chunk's window: channels 8 (u / width) .. + 7
   // at window column u % width.
   int at[kSlots], group[kSlots];  // first input position, 8-channel group
-  unsigned inside[kSlots];        // bit i: channel i of the unit is a value
+  // Windows fetched ahead of the one multiplied: a one-tap chunk is over
+  // before its successor's loads have come back.
+  constexpr int kDepth = TAPS == 1 && NT <= 2 && BUFS == 2 ? 2 : 1;
+  unsigned inside[kDepth][kSlots];  // bit i: channel i of the unit is a value
 #pragma unroll
   for (int q = 0; q < kSlots; ++q) {
     const int u = min(tid + q * kT, units - 1);
@@ -211,18 +236,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
       at[q] = m * p.view_stride + lo;
     } else {
       const int t = m + lo;
-      inside[q] = t >= 0 && t < p.len_in ? 0xFFU : 0U;
+#pragma unroll
+      for (int d = 0; d < kDepth; ++d)
+        inside[d][q] = t >= 0 && t < p.len_in ? 0xFFU : 0U;
       at[q] = min(max(t, 0), p.len_in - 1);
     }
   }
-  float xr[kSlots][8];
-  auto fetch = [&](int chunk) {
+  float window[kDepth][kSlots][8];
+  // Every wave issues the same number of loads on every path (clamped ones
+  // where there is nothing to load): the compiler then waits for the weights
+  // by counting past the window's loads instead of for all of them.
+  auto fetch = [&](int chunk, int d) __attribute__((always_inline)) {
+    auto& xr = window[d];
+    if (VIEW) {
 #pragma unroll
-    for (int q = 0; q < kSlots; ++q) {
-      if (wave * 64 + q * kT >= units)
-        break;
-      const int j = chunk * kChunk + 8 * group[q];
-      if (VIEW) {
+      for (int q = 0; q < kSlots; ++q) {
+        const int j = chunk * kChunk + 8 * group[q];
         int c = j / p.view_kernel, k = j % p.view_kernel;
         unsigned mask = 0;
 #pragma unroll
@@ -237,53 +266,70 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
             ++c;
           }
         }
-        inside[q] = mask;
-      } else {
-        const float* from = x + at[q];
-        if (j + 8 <= p.cin) {
-          from += static_cast<size_t>(j) * p.len_in;
+        inside[d][q] = mask;
+      }
+    } else if ((chunk + 1) * kChunk <= p.cin) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
-            xr[q][i] = from[static_cast<size_t>(i) * p.len_in];
-        } else {
+      for (int q = 0; q < kSlots; ++q) {
+        const float* from =
+            x + at[q] + static_cast<size_t>(chunk * kChunk + 8 * group[q]) * p.len_in;
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
-            xr[q][i] = from[static_cast<size_t>(min(j + i, p.cin - 1)) * p.len_in];
-        }
+        for (int i = 0; i < 8; ++i)
+          xr[q][i] = from[static_cast<size_t>(i) * p.len_in];
+      }
+    } else {
+#pragma unroll
+      for (int q = 0; q < kSlots; ++q) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          xr[q][i] = x[at[q] + static_cast<size_t>(min(chunk * kChunk + 8 * group[q] + i,
+                                                       p.cin - 1)) * p.len_in];
       }
     }
   };
-  auto stash = [&](int chunk, int buf) {
+  // Window d to LDS in 4 kSlots slices of two values: mask, split, and with
+  // a unit's last pair the unit's stores (past the window's units too, where
+  // nothing reads).
+  auto activate = [&](int chunk, int d) __attribute__((always_inline)) {
+    if (p.alpha_in == nullptr && p.in_act == kActNone)
+      return;
 #pragma unroll
     for (int q = 0; q < kSlots; ++q) {
-      const int u = tid + q * kT;
-      if (wave * 64 + q * kT >= units)
-        break;
       const int j = chunk * kChunk + 8 * group[q];
-      if (p.alpha_in != nullptr) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          xr[q][i] = Snake(xr[q][i], p.alpha_in[min(j + i, p.cin - 1)],
-                           SnakeInverse(p.alpha_in[min(j + i, p.cin - 1)]));
+      for (int i = 0; i < 8; ++i) {
+        const float alpha = p.alpha_in != nullptr ? p.alpha_in[min(j + i, p.cin - 1)] : 0.0F;
+        float& v = window[d][q][i];
+        if (p.alpha_in != nullptr)
+          v = Snake(v, alpha, SnakeInverse(alpha));
+        if (p.in_act == kActElu)
+          v = Elu(v);
       }
-      if (p.in_act == kActElu) {
+    }
+  };
+  uintx4 part[3];
+  unsigned mask = 0;
+  auto slice = [&](int k, int chunk, int buf, int d) __attribute__((always_inline)) {
+    const int q = k / 4, h = k % 4;
+    if (TAPS == 7 && q == kSlots - 1 && wave * 64 + q * kT >= units)
+      return;
+    if (h == 0) {
+      mask = inside[d][q];
+      const int j = chunk * kChunk + 8 * group[q];
+      if (!VIEW)
+        mask &= 0xFFU >> min(max(j + 8 - p.cin, 0), 8);
+    }
+    floatx2 rest{(mask >> 2 * h & 1U) != 0U ? window[d][q][2 * h] : 0.0F,
+                 (mask >> 2 * h & 2U) != 0U ? window[d][q][2 * h + 1] : 0.0F};
+    part[0][h] = RoundPair(rest);
+    rest = Rest(rest, part[0][h]);
+    part[1][h] = RoundPair(rest);
+    rest = Rest(rest, part[1][h]);
+    part[2][h] = RoundPair(rest);
+    if (h == 3) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          xr[q][i] = Elu(xr[q][i]);
-      }
-      unsigned mask = inside[q];
-      if (!VIEW && j + 8 > p.cin)
-        mask &= (1U << max(p.cin - j, 0)) - 1U;
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        xr[q][i] = (mask >> i & 1U) != 0U ? xr[q][i] : 0.0F;
-      uintx4 part[3];
-      Split8(xr[q], part);
-      if (u < units) {
-#pragma unroll
-        for (int s = 0; s < 3; ++s)
-          xs[(buf * 3 + s) * kMaxUnits + u] = part[s];
-      }
+      for (int s = 0; s < 3; ++s)
+        xs[(buf * 3 + s) * kMaxUnits + tid + q * kT] = part[s];
     }
   };
 
@@ -304,42 +350,89 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
       w += step_units;
   };
 
-  floatx16 main[NT] = {}, low[NT] = {};
-  uintx4 a[kAhead][3], b[2][3];
-  fetch(c_begin);
+  constexpr int kTurn = NT > 1 ? 2 : 1;  // blocks multiplied in turn
+  floatx16 main[NT] = {}, low[NT > 1 ? NT : 2] = {};
+  uintx4 a[kAhead][3], b[kTurn][3];
+#pragma unroll
+  for (int d = 0; d < kDepth; ++d)
+    fetch(min(c_begin + d, c_end - 1), d);
 #pragma unroll
   for (int i = 0; i < kAhead; ++i)
     load(a[i]);
-  for (int chunk = c_begin; chunk < c_end; ++chunk) {
-    const int buf = BUFS == 1 ? 0 : (chunk - c_begin) & 1;
-    stash(chunk, buf);
-    __syncthreads();
-    if (BUFS > 1 && chunk + 1 < c_end)
-      fetch(chunk + 1);
+  activate(c_begin, 0);
+#pragma unroll
+  for (int k = 0; k < 4 * kSlots; ++k)
+    slice(k, c_begin, 0, 0);
+  if (BUFS > 1)
+    fetch(min(c_begin + kDepth, c_end - 1), 0);
+  __syncthreads();
+  // Multiplies a chunk; with `more`, splits the next one into the other
+  // buffer between the products, whose pipe it leaves free (before them it
+  // took as long as a one-tap chunk's products), and fetches another.
+  auto multiply = [&](int chunk, int buf, bool more) __attribute__((always_inline)) {
+    const int d = kDepth == 2 ? 1 - buf : 0;
+    if (more)
+      activate(chunk + 1, d);
     const uintx4* base = xs + buf * 3 * kMaxUnits + half * width + col + l32 + shift;
-    // Block i of a chunk: column block i % NT of step i / NT.
-    auto read = [&](int i, uintx4* v) {
-      const int step = i / NT;
-      const uintx4* from =
-          base + step % kSubs * 2 * width + step / kSubs * dilation + 32 * (i % NT);
+    // Part s of blocks i kTurn .. of a chunk: column block % NT of step / NT.
+    auto read = [&](int i, int s) {
 #pragma unroll
-      for (int s = 0; s < 3; ++s)
-        v[s] = from[s * kMaxUnits];
+      for (int j = 0; j < kTurn; ++j) {
+        const int step = (i * kTurn + j) / NT;
+        b[j][s] = base[s * kMaxUnits + step % kSubs * 2 * width + step / kSubs * dilation +
+                       32 * ((i * kTurn + j) % NT)];
+      }
     };
-    read(0, b[0]);
+    read(0, 2);
+    read(0, 1);
+    read(0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    constexpr int kTurns = kSteps * NT / kTurn;
+    // The slices go behind the last two thirds of the products, when the
+    // window has arrived.
+    constexpr int kSlices = 4 * kSlots, kFrom = kTurns * 2, kOver = kTurns * 6 - kFrom;
 #pragma unroll
-    for (int i = 0; i < kSteps * NT; ++i) {
-      const int t = i % NT, step = i / NT;
-      if (i + 1 < kSteps * NT)
-        read(i + 1, b[(i + 1) & 1]);
-      // Keeps the next block's reads ahead of this block's products.
-      __builtin_amdgcn_sched_barrier(0);
-      Products(a[step % kAhead], b[i & 1], main[t], low[t]);
-      __builtin_amdgcn_sched_barrier(0);
-      if (t == NT - 1)
+    for (int i = 0; i < kTurns; ++i) {
+      const int t = i * kTurn % NT, step = i * kTurn / NT;
+      Products<kTurn>(
+          a[step % kAhead], b, main + t, low + t,
+          [&](int s) {
+            if (i + 1 < kTurns)
+              read(i + 1, s);
+          },
+          [&](int k) {
+            const int g = i * 6 + k - kFrom;
+            if (!more || g < 0)
+              return;
+#pragma unroll
+            for (int n = g * kSlices / kOver; n < (g + 1) * kSlices / kOver; ++n)
+              slice(n, chunk + 1, 1 - buf, d);
+          });
+      if (t + kTurn == NT)
         load(a[step % kAhead]);
     }
+    if (more) {
+      fetch(min(chunk + 1 + kDepth, c_end - 1), d);
+      __syncthreads();
+    }
+  };
+  if (BUFS == 1) {
+    multiply(c_begin, 0, false);
+  } else {
+    int chunk = c_begin;
+    for (; chunk + 2 < c_end; chunk += 2) {
+      multiply(chunk, 0, true);
+      multiply(chunk + 1, 1, true);
+    }
+    if (chunk + 1 < c_end) {
+      multiply(chunk, 0, true);
+      multiply(chunk + 1, 1, false);
+    } else {
+      multiply(chunk, 0, false);
+    }
   }
+  if (NT == 1)
+    low[0] += low[1];
 
   // Element r of the accumulators: output channel row + 8 (r / 4) + 4 half +
   // r % 4, position col + 32 t + l32.
@@ -407,18 +500,26 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     for (int t = 0; t < NT; ++t)
       main[t] = low[t] = floatx16{};
     const uintx4* base = xs + half * BN + col + l32;
+    static_assert(!FUSED || NT == 2, "a step is one pair of blocks");
+    auto read = [&](int step, int s) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+        b[t][s] = base[s * (BM / 8 * BN) + 2 * step * BN + 32 * t];
+    };
+    read(0, 2);
+    read(0, 1);
+    read(0, 0);
 #pragma unroll
     for (int step = 0; step < BM / 16; ++step) {
       if (step + 1 < BM / 16)
         load2(step + 1, a[(step + 1) & 1]);
-#pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        uintx4 v[3];
-#pragma unroll
-        for (int s = 0; s < 3; ++s)
-          v[s] = base[s * (BM / 8 * BN) + 2 * step * BN + 32 * t];
-        Products(a[step & 1], v, main[t], low[t]);
-      }
+      Products<kTurn>(
+          a[step & 1], b, main, low,
+          [&](int s) {
+            if (step + 1 < BM / 16)
+              read(step + 1, s);
+          },
+          [](int) {});
     }
     bias = p.bias2;
   }
@@ -573,6 +674,7 @@ __global__ __launch_bounds__(kThreads) void SplitReduceKernel(ConvParams p) {
     const int m = static_cast<int>(within % p.positions);
     const float* part = p.partial + static_cast<size_t>(rest) * p.splits * per + within;
     float v = 0.0F;
+#pragma unroll 8
     for (int s = 0; s < p.splits; ++s)
       v += part[static_cast<size_t>(s) * per];
     const int phase = rest % p.phases, batch = rest / p.phases;
@@ -646,15 +748,16 @@ void DispatchTile(const ConvParams& p, hipStream_t stream) {
            dim3(64 * WM * WN), 0, stream, true, p.splits == 1, p);
 }
 
-// Splits the input channels of a convolution whose tiles number under 256
-// until about 512 work-groups run, if there is a workspace.
-void ChooseSplits(ConvParams* p, int64_t tiles, int chunk) {
+// Splits the input channels of a convolution of `tiles` work-groups until
+// about `target` run, at least two chunks and at most `most` splits, if there
+// is a workspace.
+void ChooseSplits(ConvParams* p, int64_t tiles, int chunk, int64_t target, int most) {
   const int chunks = (p->cin + chunk - 1) / chunk;
   p->splits = 1;
   p->split_chunks = chunks;
-  if (p->partial == nullptr || tiles >= 256 || chunks < 4)
+  if (p->partial == nullptr)
     return;
-  int64_t want = std::min<int64_t>((512 + tiles - 1) / tiles, chunks / 2);
+  int64_t want = std::min<int64_t>(target / tiles, std::min(most, chunks / 2));
   const int64_t outputs = static_cast<int64_t>(p->cout) * p->positions * p->phases * p->batches;
   want = std::min<int64_t>(want, p->partial_capacity / std::max<int64_t>(outputs, 1));
   want = std::min<int64_t>(want, 65535 / (static_cast<int64_t>(p->phases) * p->batches));
@@ -676,35 +779,55 @@ int64_t Tiles(const ConvParams& p, int bm, int bn) {
   return static_cast<int64_t>((p.positions + bn - 1) / bn) * ((p.cout + bm - 1) / bm) * p.batches;
 }
 
-// The tile: all output channels of a narrow layer (32 x 256 when the input is
-// one chunk, so that two work-groups' windows fit a CU's LDS, else 32 x 128;
-// 64 x 128), else 128 x 128 where that gives every CU a work-group, else
-// 128 x 64.
+// The tile and the splits. All output channels of a narrow layer: 32 x 256
+// when the input is one chunk, so that two work-groups' windows fit a CU's
+// LDS, else 32 x 128; 64 x 128; about 512 work-groups.
+//
+// Wider layers take 128 x 64, or 128 x 32 while that leaves CUs idle; a split
+// costs a pass of partial sums, so it only has to give each CU one work-group,
+// unless the sums are so long (over 512 channels x 7 taps) that three balance
+// better. Measured at one tap, 768 -> 3072 channels: 500 positions 20.6 us at
+// 384 tiles of 128 x 32, 21.3 at 192 of 128 x 64, 29-30 split in two; 1046
+// positions 39.2 and 34.5 (408 tiles of 128 x 64); 768 -> 768 at 150
+// positions 15.0 at 30 tiles, 11.9 and 10.7 split in two and three. At seven
+// taps: 512 channels x 2000 positions 63.6 at 128 tiles of 128 x 64, 43.4,
+// 44.9, 48.0 split in two, four, six; x 200 positions 16.4 (16 tiles, eight
+// splits) and 13.8 (28 tiles of 128 x 32, eight); 1024 x 750 65.7 at two
+// splits of 96 tiles, 57.8 at five, 54.3 at eight. 128 x 128 tiles were
+// slower at every size (512 x 12000, seven taps: 191 to 160).
 template <int TAPS, ConvKind KIND>
 void DispatchTaps(const ConvParams& params, hipStream_t stream) {
   ConvParams p = params;
-  const bool wide = p.cout > 64 && Tiles(p, 128, 128) >= 256;
-  const bool one = p.cin <= 32;
-  const int columns = p.cout <= 32 ? (one ? 256 : 128) : p.cout <= 64 || wide ? 128 : 64;
-  ChooseSplits(&p, Tiles(p, p.cout <= 32 ? 32 : p.cout <= 64 ? 64 : 128, columns),
-               TileChunk(TAPS, columns));
-  if (p.cout <= 32 && one)
-    DispatchTile<1, 4, 2, TAPS, 1, KIND>(p, stream);
-  else if (p.cout <= 32)
-    DispatchTile<1, 4, 1, TAPS, 2, KIND>(p, stream);
-  else if (p.cout <= 64)
-    DispatchTile<2, 2, 2, TAPS, 2, KIND>(p, stream);
-  else if (wide)
-    DispatchTile<4, 1, 4, TAPS, 2, KIND>(p, stream);
-  else
-    DispatchTile<4, 1, 2, TAPS, 2, KIND>(p, stream);
+  if (p.cout <= 64) {
+    const bool one = p.cin <= 32;
+    const int rows = p.cout <= 32 ? 32 : 64, columns = rows == 32 && one ? 256 : 128;
+    const int64_t tiles = Tiles(p, rows, columns);
+    ChooseSplits(&p, tiles, TileChunk(TAPS, columns), tiles < 256 ? 512 + tiles - 1 : 1, 65535);
+    if (rows == 32 && one)
+      DispatchTile<1, 4, 2, TAPS, 1, KIND>(p, stream);
+    else if (rows == 32)
+      DispatchTile<1, 4, 1, TAPS, 2, KIND>(p, stream);
+    else
+      DispatchTile<2, 2, 2, TAPS, 2, KIND>(p, stream);
+  } else {
+    const int64_t tiles = Tiles(p, 128, 64);
+    const int most = TAPS == 7 ? 8 : 65535;
+    const bool wide = TAPS == 1 ? tiles >= 400
+                                : tiles * std::min(most, (p.cin + 31) / 32 / 2) >= 256;
+    ChooseSplits(&p, wide ? tiles : Tiles(p, 128, 32), TileChunk(TAPS, wide ? 64 : 32),
+                 TAPS == 7 && p.cin > 512 ? 768 : 256, most);
+    if (wide)
+      DispatchTile<4, 1, 2, TAPS, 2, KIND>(p, stream);
+    else
+      DispatchTile<4, 1, 1, TAPS, 2, KIND>(p, stream);
+  }
   Reduce(p, stream);
 }
 
 // A residual unit of up to 128 channels in one launch.
 void DispatchFused(const ConvParams& params, hipStream_t stream) {
   ConvParams p = params;
-  ChooseSplits(&p, 256, 32);
+  ChooseSplits(&p, 1, 32, 1, 1);
   if (p.cout <= 32)
     DispatchTile<1, 4, 2, 7, 1, kFused>(p, stream);
   else if (p.cout <= 64)
@@ -716,7 +839,8 @@ void DispatchFused(const ConvParams& params, hipStream_t stream) {
 // A transposed convolution: a wave per phase.
 void DispatchUp(const ConvParams& params, hipStream_t stream) {
   ConvParams p = params;
-  ChooseSplits(&p, Tiles(p, 32, 64), 32);
+  const int64_t tiles = Tiles(p, 32, 64);
+  ChooseSplits(&p, tiles, 32, tiles < 256 ? 512 + tiles - 1 : 1, 65535);
   switch (p.phases) {
     case 2: DispatchTile<2, 1, 2, 2, 2, kUp>(p, stream); break;
     case 3: DispatchTile<3, 1, 2, 2, 2, kUp>(p, stream); break;

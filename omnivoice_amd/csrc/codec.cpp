@@ -413,7 +413,6 @@ void CodecEngine::Enqueue(const std::int32_t* codes, std::int64_t frames, float*
   // Output convolution of snake(x), no tanh (codec.cpp:244-251).
   OutputConvParams o{};
   o.x = xa_[cur].get();
-  o.alpha = nullptr;
   o.w = out_w_.get();
   o.bias = out_b_.get();
   o.y = audio;

@@ -91,11 +91,9 @@ struct ConvParams {
 void LaunchConv(const ConvParams& p, hipStream_t stream);
 
 // The decoder's last layer, one output channel: y[t] = bias + sum_{k, i}
-// w[k][i] act(x[i][t + k - pad]), pad = (taps - 1) / 2, act the Snake of
-// `alpha` or the identity when it is null.
+// w[k][i] x[i][t + k - pad], pad = (taps - 1) / 2.
 struct OutputConvParams {
   const float* x;      // [cin][length]
-  const float* alpha;  // [cin] or null
   const float* w;      // [taps][cin]
   const float* bias;   // [1]
   float* y;            // [length]

@@ -17,8 +17,7 @@ namespace ovg {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kOutTile = 256;  // samples per work-group of the output conv
-constexpr int kOutChunk = 32;  // input channels per chunk of the output conv
+constexpr int kOutTile = kThreads;  // samples per work-group of the output conv
 
 // kernels/codec_kernels.hip:20-22 of the reference: v + sin^2(a v) / (a + 1e-9),
 // with 1 / (a + 1e-9) given. x = a v less its nearest multiple of pi (pi in
@@ -115,13 +114,13 @@ constexpr int TileChunk(int taps, int columns) {
 
 // One float32 convolution as an implicit GEMM over bf16 triples (split.hpp):
 // rows are output channels, columns output positions, the sum runs over
-// chunks of 32 or 64 input channels x taps in steps of 16 channels. A wave owns 32
-// rows x NT blocks of 32 columns, WM x WN waves a work-group.
+// chunks of 32 to 128 input channels x taps in steps of 16 channels. A wave
+// owns 32 rows x NT blocks of 32 columns, WM x WN waves a work-group.
 //
 // The weights come split and in step order from memory (PackConvWeights):
 // each wave reads its own rows' 16-byte operands straight into registers
-// some 1500 cycles of products ahead, so they cost no LDS traffic and no barrier; with all waves on
-// one row block of columns (WN = 1) nothing is read twice. The chunk's input
+// kAhead steps ahead, so they cost no LDS traffic and no barrier; with all
+// waves on the same columns (WN = 1) nothing is read twice. The chunk's input
 // window (the tile's positions plus the taps' spread) is fetched as float32
 // while the previous chunk is multiplied, split once per work-group on its
 // way to LDS as [part][8 channels][position] 16-byte units, and every tap
@@ -687,40 +686,57 @@ __global__ __launch_bounds__(kThreads) void SplitReduceKernel(ConvParams p) {
   }
 }
 
+// Four outputs a thread from a register window of 4 + taps - 1 samples per
+// channel, read in 16-byte runs whose overlaps stay in the caches; the waves
+// of a work-group take a quarter of the channels each, eight in flight, and
+// meet in LDS. Bound by memory at long signals (with a work-group's window in
+// LDS and one read per product 60 s of 32 channels, 184 MB, took 131 us), by
+// one round trip to it at short ones.
+template <int TAPS>
 __global__ __launch_bounds__(kThreads) void OutputConvKernel(OutputConvParams p) {
-  __shared__ float xs[kOutChunk][kOutTile + kConvMaxTaps - 1];
-  const int tid = threadIdx.x;
-  const int t0 = blockIdx.x * kOutTile;
-  const int pad = (p.taps - 1) / 2;
-  const int width = kOutTile + p.taps - 1;
-  float acc = 0.0F;
-  for (int c0 = 0; c0 < p.cin; c0 += kOutChunk) {
-    for (int j = tid; j < width; j += kThreads) {
-      const int t = t0 - pad + j;
-      const bool inside = t >= 0 && t < p.length;
-      const int tc = min(max(t, 0), p.length - 1);
-      float v[kOutChunk];
+  constexpr int kPad = (TAPS - 1) / 2, kRuns = (4 + TAPS - 1 + 3) / 4;
+  constexpr int kWaves = kThreads / 64;
+  __shared__ floatx4 sums[kWaves][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t0 = blockIdx.x * kOutTile + lane * 4;
+  const int per = (p.cin + kWaves - 1) / kWaves;
+  const int c_end = min(p.cin, (wave + 1) * per);
+  const bool inside = t0 >= kPad && t0 - kPad + 4 * kRuns <= p.length;
+  floatx4 sum = {0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll 8
+  for (int c = wave * per; c < c_end; ++c) {
+    const float* row = p.x + static_cast<size_t>(c) * p.length;
+    float v[4 * kRuns];
+    if (inside) {
 #pragma unroll
-      for (int c = 0; c < kOutChunk; ++c)
-        v[c] = p.x[static_cast<size_t>(min(c0 + c, p.cin - 1)) * p.length + tc];
+      for (int r = 0; r < kRuns; ++r)
+        *reinterpret_cast<floatx4*>(v + 4 * r) =
+            *reinterpret_cast<const Unaligned4*>(row + t0 - kPad + 4 * r);
+    } else {
 #pragma unroll
-      for (int c = 0; c < kOutChunk; ++c)
-        xs[c][j] = inside && c0 + c < p.cin
-                       ? (p.alpha != nullptr ? Snake(v[c], p.alpha[min(c0 + c, p.cin - 1)],
-                                                     SnakeInverse(p.alpha[min(c0 + c, p.cin - 1)]))
-                                             : v[c])
-                       : 0.0F;
+      for (int i = 0; i < 4 * kRuns; ++i) {
+        const int t = t0 - kPad + i;
+        const float sample = row[min(max(t, 0), p.length - 1)];
+        v[i] = t >= 0 && t < p.length ? sample : 0.0F;
+      }
     }
-    __syncthreads();
-    const int channels = min(kOutChunk, p.cin - c0);
-    for (int c = 0; c < channels; ++c)
-      for (int k = 0; k < p.taps; ++k)
-        acc += p.w[k * p.cin + c0 + c] * xs[c][tid + k];
-    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < TAPS; ++k)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        sum[e] += p.w[k * p.cin + c] * v[e + k];
   }
-  const int t = t0 + tid;
-  if (t < p.length)
-    p.y[t] = acc + p.bias[0];
+  sums[wave][lane] = sum;
+  __syncthreads();
+  const int t = blockIdx.x * kOutTile + threadIdx.x;
+  if (t < p.length) {
+    float v = 0.0F;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+      v += sums[w][threadIdx.x / 4][threadIdx.x % 4];
+    p.y[t] = v + p.bias[0];
+  }
 }
 
 __global__ __launch_bounds__(kThreads) void RvqKernel(RvqParams p) {
@@ -933,8 +949,16 @@ void LaunchOutputConv(const OutputConvParams& p, hipStream_t stream) {
   Require(p.cin >= 1 && p.length >= 1, "output conv: empty shape");
   Require(p.taps >= 1 && p.taps <= kConvMaxTaps && p.taps % 2 == 1,
           "output conv: 1, 3, 5 or 7 taps");
-  Dispatch(OutputConvKernel, dim3((p.length + kOutTile - 1) / kOutTile), dim3(kThreads), 0,
-           stream, true, true, p);
+  const dim3 grid(static_cast<unsigned>((p.length + int64_t{kOutTile} - 1) / kOutTile));
+  auto launch = [&](auto* kernel) {
+    Dispatch(kernel, grid, dim3(kThreads), 0, stream, true, true, p);
+  };
+  switch (p.taps) {
+    case 1: launch(OutputConvKernel<1>); break;
+    case 3: launch(OutputConvKernel<3>); break;
+    case 5: launch(OutputConvKernel<5>); break;
+    default: launch(OutputConvKernel<7>); break;
+  }
 }
 
 void LaunchRvq(const RvqParams& p, hipStream_t stream) {

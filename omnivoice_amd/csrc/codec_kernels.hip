@@ -140,7 +140,7 @@ constexpr int TileChunk(int taps, int columns) {
 // work draws) at 128 channels and more; at 32 and 64 by them, the activations'
 // vector work and memory alike. At a 60 s signal: the k7 convolutions of 256
 // and 512 channels 200 TFLOP/s of float32 products (87 on the float32 matrix
-// cores), a residual unit of 128 / 64 / 32 channels 400 / 273 / 300 us where
+// cores), a residual unit of 128 / 64 / 32 channels 399 / 272 / 282 us where
 // its two launches took 492 / 329 / 397, the transposed convolutions 204 us
 // a launch where one phase per work-group, its outputs scattered, took 295.
 // Splitting a chunk between its predecessor's products instead of before its
@@ -499,7 +499,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     for (int t = 0; t < NT; ++t)
       main[t] = low[t] = floatx16{};
     const uintx4* base = xs + half * BN + col + l32;
-    static_assert(!FUSED || NT == 2, "a step is one pair of blocks");
+    static_assert(!FUSED || NT == kTurn, "a step is one turn of blocks");
+    if (NT == 1)
+      low[1] = floatx16{};
     auto read = [&](int step, int s) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
@@ -520,6 +522,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
           },
           [](int) {});
     }
+    if (NT == 1)
+      low[0] += low[1];
     bias = p.bias2;
   }
 
@@ -840,14 +844,23 @@ void DispatchTaps(const ConvParams& params, hipStream_t stream) {
   Reduce(p, stream);
 }
 
-// A residual unit of up to 128 channels in one launch.
+// A residual unit of up to 128 channels in one launch. Half the columns where
+// the wider tile leaves CUs idle: 24000 samples of 32 channels 18.5 -> 13.3 us,
+// 8000 of 64 22.3 -> 16.8, 4000 of 128 29.9 -> 23.3; at 60 s the wider tile is
+// 15-25 % faster, but for the one chunk of 32 channels, where the narrow one
+// leaves LDS for more work-groups (301 -> 282 us).
 void DispatchFused(const ConvParams& params, hipStream_t stream) {
   ConvParams p = params;
   ChooseSplits(&p, 1, 32, 1, 1);
+  const auto few = [&](int columns) { return Tiles(p, 128, columns) < 256; };
   if (p.cout <= 32)
-    DispatchTile<1, 4, 2, 7, 1, kFused>(p, stream);
+    DispatchTile<1, 4, 1, 7, 1, kFused>(p, stream);
+  else if (p.cout <= 64 && few(128))
+    DispatchTile<2, 2, 1, 7, 2, kFused>(p, stream);
   else if (p.cout <= 64)
     DispatchTile<2, 2, 2, 7, 2, kFused>(p, stream);
+  else if (few(64))
+    DispatchTile<4, 1, 1, 7, 2, kFused>(p, stream);
   else
     DispatchTile<4, 1, 2, 7, 2, kFused>(p, stream);
 }

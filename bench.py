@@ -38,7 +38,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP16_TFLOPS = 2500.0  # MI355X dense fp16 MFMA
-PEAK_FP32_TFLOPS = 157.3   # MI355X dense fp32 MFMA
+PEAK_FP32_TFLOPS = PEAK_FP16_TFLOPS / 6  # a float32 product is six bf16 ones (split.hpp)
 PEAK_HBM_GBS = 8000.0      # MI355X HBM3E
 
 WORKLOADS = {

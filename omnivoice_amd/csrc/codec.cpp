@@ -10,10 +10,10 @@
 //    table[c][e][o] = sum_h fc2[o][h] (embed_c project_c^T + bias_c)[e][h],
 //    so decoding starts with one gather-sum of codebook rows per frame
 //    instead of a table gather and a GEMM.
-//  * Every convolution is one kernel: the Snake activation of its input is
-//    applied while the input is staged, bias and residual addition in the
-//    epilogue. A transposed convolution of stride s runs as s output phases
-//    of a two-tap convolution instead of a GEMM into columns plus col2im.
+//  * Every convolution is one kernel, its Snake, bias and residual addition in
+//    the epilogue; a residual unit of up to 128 channels is one kernel too. A
+//    transposed convolution of stride s runs as s output phases of a two-tap
+//    convolution, a wave per phase, instead of a GEMM into columns plus col2im.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

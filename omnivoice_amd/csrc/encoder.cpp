@@ -8,7 +8,7 @@
 //
 // Layout: every signal is channel-major ([channels][positions]), HuBERT's
 // hidden states included ([width][steps]), so that every GEMM-shaped layer
-// is a convolution on the fp32 matrix cores (codec_kernels.hip):
+// is a convolution on the matrix cores (codec_kernels.hip):
 //  * a linear layer is a one-tap convolution;
 //  * a strided, long or grouped convolution reads its input through a strided
 //    window (ConvParams::view_kernel), a one-tap convolution of channels x taps;

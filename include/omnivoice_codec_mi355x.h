@@ -107,6 +107,31 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length,
                             int64_t out, int64_t stride, float* y, void* stream,
                             char* error, size_t error_len);
 
+/* A strided, grouped or split convolution for op-level tests: x [in][length]
+ * and y [out][positions] in device memory; w [out][in / groups][kernel] and
+ * b [out] on the host; ELU on the input when elu is set. One group of 1, 2
+ * or 7 taps at stride 1 with padding (kernel - 1) dilation / 2 on each side
+ * and as many outputs as inputs runs tap by tap, everything else (dilation
+ * 1) through a strided window of the input. `split_floats` is the size of a
+ * workspace with which the input channels may be split (0: none).
+ * Synchronises `stream`. */
+int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length,
+                          const float* w, const float* b, int64_t out,
+                          int64_t kernel, int64_t dilation, int64_t stride,
+                          int64_t padding, int64_t groups, int elu,
+                          int64_t split_floats, float* y, int64_t positions,
+                          void* stream, char* error, size_t error_len);
+
+/* A residual unit of up to 128 channels for op-level tests: y += w2
+ * snake(w1 x + b1) + b2, w1 [channels][channels][7] at `dilation`, w2
+ * [channels][channels], b1 and b2 on the host; x (its Snake already applied)
+ * and y [channels][length] and alpha [channels] in device memory.
+ * Synchronises `stream`. */
+int ovc_op_residual_unit(const float* x, int64_t channels, int64_t length,
+                         const float* w1, const float* b1, int64_t dilation,
+                         const float* alpha, const float* w2, const float* b2,
+                         float* y, void* stream, char* error, size_t error_len);
+
 /* ------------------------------------------------------------ the encoder */
 
 /* The encoder's dimensions: CodecConfig's frame_samples and
@@ -186,6 +211,25 @@ int ovc_encode_device(ovc_encoder* handle, const float* samples, int64_t length,
 int ovc_profile_encode(ovc_encoder* handle, int64_t length, int64_t repeats,
                        ovg_kernel_stat* stats, int64_t capacity, int64_t* count,
                        char* error, size_t error_len);
+
+/* The encoder's attention for op-level tests: q, k, v and out
+ * [heads][head_dim][steps] in device memory, out[d][t] = sum_s v[d][s]
+ * softmax_s(scale sum_e k[e][s] q[e][t]). Synchronises `stream`. */
+int ovc_op_head_attention(const float* q, const float* k, const float* v,
+                          int64_t heads, int64_t head_dim, int64_t steps,
+                          float scale, float* out, void* stream, char* error,
+                          size_t error_len);
+
+/* The residual vector quantizer for op-level tests: x [hidden][frames] and
+ * codes [stages][frames] in device memory; project [stages][dim][hidden],
+ * bias [stages][dim], embed [stages][entries][dim] and table
+ * [stages][entries][hidden] (the rows subtracted) on the host. Synchronises
+ * `stream`. */
+int ovc_op_quantize(const float* x, int64_t hidden, int64_t frames,
+                    const float* project, const float* bias, const float* embed,
+                    const float* table, int64_t stages, int64_t dim,
+                    int64_t entries, int32_t* codes, void* stream, char* error,
+                    size_t error_len);
 
 #ifdef __cplusplus
 }

@@ -155,6 +155,11 @@ EXPORTS = {
                                      ctypes.c_int, _ptr, _ptr, _err, _sz]),
     "ovc_op_conv_transpose1d": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr, _i64,
                                                _i64, _ptr, _ptr, _err, _sz]),
+    "ovc_op_conv1d_strided": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _i64, _i64, _i64,
+                                             _i64, _i64, _i64, ctypes.c_int, _i64, _ptr, _i64,
+                                             _ptr, _err, _sz]),
+    "ovc_op_residual_unit": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _i64, _ptr, _ptr,
+                                            _ptr, _ptr, _ptr, _err, _sz]),
     # the audio encoder (include/omnivoice_codec_mi355x.h)
     "ovc_encoder_create": (ctypes.c_int, [ctypes.POINTER(_EncoderConfig), ctypes.c_char_p,
                                           _u64, ctypes.POINTER(_ptr), _err, _sz]),
@@ -166,6 +171,10 @@ EXPORTS = {
     "ovc_encode_device": (ctypes.c_int, [_ptr, _ptr, _i64, _ptr, _ptr, _err, _sz]),
     "ovc_profile_encode": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _i64,
                                           ctypes.POINTER(_i64), _err, _sz]),
+    "ovc_op_head_attention": (ctypes.c_int, [_ptr, _ptr, _ptr, _i64, _i64, _i64, _f32, _ptr,
+                                             _ptr, _err, _sz]),
+    "ovc_op_quantize": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr, _i64, _i64,
+                                       _i64, _ptr, _ptr, _err, _sz]),
 }
 
 _lib: Optional[ctypes.CDLL] = None
@@ -750,6 +759,30 @@ def op_conv_transpose1d(x, w, b, y, stride: int, alpha=None, stream=None) -> Non
                                          _stream(stream), err, len(err)), err)
 
 
+def op_conv1d_strided(x, w, b, y, dilation: int = 1, stride: int = 1, padding: int = 0,
+                      groups: int = 1, elu: bool = False, split_floats: int = 0,
+                      stream=None) -> None:
+    """x [in][L] and y [out][positions]: float32 device tensors; w
+    [out][in / groups][k] and b [out]: host float32 arrays."""
+    w = np.ascontiguousarray(w, dtype=np.float32)
+    b = np.ascontiguousarray(b, dtype=np.float32)
+    err = _buf()
+    _check(lib().ovc_op_conv1d_strided(_dev(x), x.shape[0], x.shape[1], _p(w), _p(b), w.shape[0],
+                                       w.shape[2], dilation, stride, padding, groups, int(elu),
+                                       split_floats, _dev(y), y.shape[1], _stream(stream), err,
+                                       len(err)), err)
+
+
+def op_residual_unit(x, w1, b1, alpha, w2, b2, y, dilation: int = 1, stream=None) -> None:
+    """y += w2 snake(w1 x + b1) + b2; x, y [c][L] and alpha [c]: float32 device
+    tensors; w1 [c][c][7], w2 [c][c], b1 and b2 [c]: host float32 arrays."""
+    w1, b1, w2, b2 = (np.ascontiguousarray(a, dtype=np.float32) for a in (w1, b1, w2, b2))
+    err = _buf()
+    _check(lib().ovc_op_residual_unit(_dev(x), x.shape[0], x.shape[1], _p(w1), _p(b1), dilation,
+                                      _dev(alpha), _p(w2), _p(b2), _dev(y), _stream(stream), err,
+                                      len(err)), err)
+
+
 # --------------------------------------------------------------- audio encoder
 
 def encoder_released_config() -> dict:
@@ -868,3 +901,24 @@ class Encoder:
             self.close()
         except Exception:
             pass
+
+
+def op_head_attention(q, k, v, out, scale: float, stream=None) -> None:
+    """q, k, v, out: float32 device tensors [heads][head_dim][steps]."""
+    err = _buf()
+    _check(lib().ovc_op_head_attention(_dev(q), _dev(k), _dev(v), *q.shape, scale, _dev(out),
+                                       _stream(stream), err, len(err)), err)
+
+
+def op_quantize(x, project, bias, embed, table, codes, stream=None) -> None:
+    """x [hidden][frames] (float32) and codes [stages][frames] (int32): device
+    tensors; project [stages][dim][hidden], bias [stages][dim], embed
+    [stages][entries][dim], table [stages][entries][hidden]: host float32
+    arrays."""
+    project, bias, embed, table = (np.ascontiguousarray(a, dtype=np.float32)
+                                   for a in (project, bias, embed, table))
+    stages, entries, dim = embed.shape
+    err = _buf()
+    _check(lib().ovc_op_quantize(_dev(x), x.shape[0], x.shape[1], _p(project), _p(bias),
+                                 _p(embed), _p(table), stages, dim, entries, _dev(codes),
+                                 _stream(stream), err, len(err)), err)

@@ -660,4 +660,114 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length, const fl
   });
 }
 
+int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length, const float* w,
+                          const float* b, int64_t out, int64_t kernel, int64_t dilation,
+                          int64_t stride, int64_t padding, int64_t groups, int elu,
+                          int64_t split_floats, float* y, int64_t positions, void* stream,
+                          char* error, size_t error_len) {
+  return CodecGuard("conv1d_strided: ", error, error_len, [&] {
+    ovg::Require(x && w && b && y, "null pointer");
+    const int64_t limit = int64_t{1} << 31;
+    for (const int64_t n : {in, out, length, kernel, dilation, stride, groups, positions})
+      ovg::Require(n >= 1 && n < limit, "bad shape");
+    ovg::Require(in % groups == 0 && out % groups == 0 && in * out < limit &&
+                     in * out / groups * kernel < limit && padding >= 0 && padding < limit &&
+                     split_floats >= 0 && split_floats < limit &&
+                     (positions - 1) * stride + (kernel - 1) * dilation <
+                         length + 2 * padding,
+                 "bad shape");
+    const bool taps = stride == 1 && groups == 1 && positions == length &&
+                      (kernel == 1 || kernel == 2 || kernel == 7) &&
+                      padding == (kernel - 1) * dilation / 2;
+    ovg::Require(taps || dilation == 1, "a strided or grouped convolution is not dilated");
+    const int K = static_cast<int>(kernel), G = static_cast<int>(groups);
+    const int I = static_cast<int>(in) / G, O = static_cast<int>(out) / G;
+    std::vector<float> layout;
+    const std::size_t per = static_cast<std::size_t>(O) * I * K;
+    for (int g = 0; g < G; ++g) {
+      const std::vector<float> one(w + g * per, w + (g + 1) * per);
+      const auto turned = taps ? ovg::ConvLayout(one, O, I, K) : ovg::ConvLayout(one, O, I * K, 1);
+      layout.insert(layout.end(), turned.begin(), turned.end());
+    }
+    ovg::DeviceBuffer<ovg::ConvUnit> wd;
+    ovg::DeviceBuffer<float> bd, partial;
+    if (taps)
+      ovg::UploadConv(wd, layout, 1, K, I, O);
+    else
+      ovg::UploadConv(wd, layout, G, 1, I * K, O);
+    ovg::Upload(bd, std::vector<float>(b, b + out));
+    partial.Reserve(static_cast<std::size_t>(split_floats));
+    ovg::ConvParams p{};
+    p.x = x;
+    p.w = wd.get();
+    p.bias = bd.get();
+    p.y = y;
+    p.cin = taps ? I : I * K;
+    p.len_in = static_cast<int>(length);
+    p.cout = O;
+    p.len_out = p.positions = static_cast<int>(positions);
+    p.taps = taps ? K : 1;
+    p.phases = 1;
+    p.dilation = static_cast<int>(dilation);
+    p.first[0] = -static_cast<int>(padding);
+    if (!taps) {
+      p.view_kernel = K;
+      p.view_stride = static_cast<int>(stride);
+      p.channels = I;
+      p.batches = G;
+      p.x_batch = static_cast<int64_t>(I) * length;
+      p.b_batch = O;
+      p.y_batch = static_cast<int64_t>(O) * positions;
+    }
+    p.in_act = elu ? ovg::kActElu : ovg::kActNone;
+    p.partial = split_floats > 0 ? partial.get() : nullptr;
+    p.partial_capacity = split_floats;
+    auto s = static_cast<hipStream_t>(stream);
+    ovg::LaunchConv(p, s);
+    ovg::Check(hipStreamSynchronize(s), "conv1d_strided");
+    return OVG_OK;
+  });
+}
+
+int ovc_op_residual_unit(const float* x, int64_t channels, int64_t length, const float* w1,
+                         const float* b1, int64_t dilation, const float* alpha, const float* w2,
+                         const float* b2, float* y, void* stream, char* error,
+                         size_t error_len) {
+  return CodecGuard("residual_unit: ", error, error_len, [&] {
+    ovg::Require(x && w1 && b1 && alpha && w2 && b2 && y, "null pointer");
+    ovg::Require(channels >= 1 && channels <= ovg::kConvFusedChannels && length >= 1 &&
+                     dilation >= 1 && dilation <= ovg::kConvMaxSpan &&
+                     channels * length < (int64_t{1} << 31),
+                 "bad shape");
+    const int C = static_cast<int>(channels);
+    const std::size_t square = static_cast<std::size_t>(C) * C;
+    ovg::DeviceBuffer<ovg::ConvUnit> wd1, wd2;
+    ovg::DeviceBuffer<float> bd1, bd2;
+    ovg::UploadConv(wd1, ovg::ConvLayout(std::vector<float>(w1, w1 + 7 * square), C, C, 7), 1, 7,
+                    C, C);
+    ovg::UploadConv(wd2, ovg::ConvLayout(std::vector<float>(w2, w2 + square), C, C, 1), 1, 1, C,
+                    C);
+    ovg::Upload(bd1, std::vector<float>(b1, b1 + C));
+    ovg::Upload(bd2, std::vector<float>(b2, b2 + C));
+    ovg::ConvParams p{};
+    p.x = x;
+    p.w = wd1.get();
+    p.bias = bd1.get();
+    p.w2 = wd2.get();
+    p.bias2 = bd2.get();
+    p.alpha_mid = alpha;
+    p.residual = p.y = y;
+    p.cin = p.cout = C;
+    p.len_in = p.len_out = p.positions = static_cast<int>(length);
+    p.taps = 7;
+    p.phases = 1;
+    p.dilation = static_cast<int>(dilation);
+    p.first[0] = -3 * p.dilation;
+    auto s = static_cast<hipStream_t>(stream);
+    ovg::LaunchConv(p, s);
+    ovg::Check(hipStreamSynchronize(s), "residual_unit");
+    return OVG_OK;
+  });
+}
+
 }  // extern "C"

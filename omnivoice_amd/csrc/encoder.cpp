@@ -118,7 +118,23 @@ struct Stage {
   DeviceBuffer<float> project, bias;  // [hidden][dim], [dim]
   DeviceBuffer<float> embed, table;   // [dim][entries], [entries][hidden]
   DeviceBuffer<double> norms;         // [entries]
+  RvqStage params() const {
+    return {project.get(), bias.get(), embed.get(), norms.get(), table.get()};
+  }
 };
+std::unique_ptr<Stage> MakeStage(const std::vector<float>& project,  // [dim][hidden]
+                                 const std::vector<float>& bias,
+                                 const std::vector<float>& embed,  // [entries][dim]
+                                 const std::vector<float>& table, const std::vector<double>& norms,
+                                 int dim, int hidden, int entries) {
+  auto st = std::make_unique<Stage>();
+  Upload(st->project, ConvLayout(project, dim, hidden, 1));
+  Upload(st->bias, bias);
+  Upload(st->embed, ConvLayout(embed, entries, dim, 1));
+  Upload(st->table, table);
+  Upload(st->norms, norms);
+  return st;
+}
 
 // Shapes of one encode of `length` samples.
 struct Plan {
@@ -438,15 +454,8 @@ EncoderEngine::EncoderEngine(const ovc_encoder_config& cfg, std::uint64_t seed,
     w.join();
   std::vector<RvqStage> stage_list;
   for (int q = 0; q < cfg.codebooks; ++q) {
-    auto st = std::make_unique<Stage>();
-    Upload(st->project, ConvLayout(pw[q], D, H, 1));
-    Upload(st->bias, pb[q]);
-    Upload(st->embed, ConvLayout(emb[q], E, D, 1));
-    Upload(st->table, tables[q]);
-    Upload(st->norms, norms[q]);
-    stage_list.push_back({st->project.get(), st->bias.get(), st->embed.get(), st->norms.get(),
-                          st->table.get()});
-    stages_[q] = std::move(st);
+    stages_[q] = MakeStage(pw[q], pb[q], emb[q], tables[q], norms[q], D, H, E);
+    stage_list.push_back(stages_[q]->params());
   }
   Upload(stage_list_, stage_list);
   partial_.Reserve(kPartialFloats);
@@ -1084,6 +1093,71 @@ int ovc_profile_encode(ovc_encoder* handle, int64_t length, int64_t repeats,
       ++n;
     }
     *count = n;
+    return OVG_OK;
+  });
+}
+
+int ovc_op_head_attention(const float* q, const float* k, const float* v, int64_t heads,
+                          int64_t head_dim, int64_t steps, float scale, float* out,
+                          void* stream, char* error, size_t error_len) {
+  return ovg::CodecGuard("head_attention: ", error, error_len, [&] {
+    const int64_t limit = int64_t{1} << 31;
+    ovg::Require(heads >= 1 && heads < limit && head_dim >= 1 && head_dim < limit && steps >= 1 &&
+                     steps < limit && heads * head_dim < limit &&
+                     heads * head_dim * steps < limit,
+                 "bad shape");
+    const int H = static_cast<int>(heads), D = static_cast<int>(head_dim),
+              T = static_cast<int>(steps);
+    ovg::DeviceBuffer<std::uint16_t> packed;
+    packed.Reserve(ovg::PackedHeadsElements(H, D, T));
+    auto s = static_cast<hipStream_t>(stream);
+    ovg::LaunchHeadAttention({q, k, v, out, packed.get(), H, D, T, scale}, s);
+    ovg::Check(hipStreamSynchronize(s), "head_attention");
+    return OVG_OK;
+  });
+}
+
+int ovc_op_quantize(const float* x, int64_t hidden, int64_t frames, const float* project,
+                    const float* bias, const float* embed, const float* table, int64_t stages,
+                    int64_t dim, int64_t entries, int32_t* codes, void* stream, char* error,
+                    size_t error_len) {
+  return ovg::CodecGuard("quantize: ", error, error_len, [&] {
+    ovg::Require(x && project && bias && embed && table && codes, "null pointer");
+    const int64_t limit = int64_t{1} << 31;
+    for (const int64_t n : {hidden, frames, stages, dim, entries})
+      ovg::Require(n >= 1 && n < limit, "bad shape");
+    ovg::Require(hidden * frames < limit && dim * hidden < limit && entries * hidden < limit &&
+                     entries * dim < limit && stages <= 1024,
+                 "bad shape");
+    const int H = static_cast<int>(hidden), F = static_cast<int>(frames),
+              D = static_cast<int>(dim), E = static_cast<int>(entries);
+    std::vector<std::unique_ptr<ovg::Stage>> held;
+    std::vector<ovg::RvqStage> list;
+    for (int64_t q = 0; q < stages; ++q) {
+      const float* rows = embed + q * E * D;
+      std::vector<double> norms(E, 0.0);
+      for (int e = 0; e < E; ++e)
+        for (int d = 0; d < D; ++d)
+          norms[e] += static_cast<double>(rows[static_cast<std::size_t>(e) * D + d]) *
+                      rows[static_cast<std::size_t>(e) * D + d];
+      const float* proj = project + q * D * H;
+      const float* sub = table + q * E * H;
+      held.push_back(ovg::MakeStage(
+          std::vector<float>(proj, proj + static_cast<std::size_t>(D) * H),
+          std::vector<float>(bias + q * D, bias + (q + 1) * D),
+          std::vector<float>(rows, rows + static_cast<std::size_t>(E) * D),
+          std::vector<float>(sub, sub + static_cast<std::size_t>(E) * H), norms, D, H, E));
+      list.push_back(held.back()->params());
+    }
+    ovg::DeviceBuffer<ovg::RvqStage> device;
+    ovg::Upload(device, list);
+    ovg::DeviceBuffer<float> residual;
+    residual.Reserve(static_cast<std::size_t>(hidden * frames));
+    auto s = static_cast<hipStream_t>(stream);
+    ovg::LaunchRvqEncode({x, device.get(), residual.get(), codes, static_cast<int>(stages), D, E,
+                          H, F},
+                         s);
+    ovg::Check(hipStreamSynchronize(s), "quantize");
     return OVG_OK;
   });
 }

@@ -120,10 +120,99 @@ def test_conv_transpose1d_tile_edges(cin, cout, length, stride):
     assert (np.abs(y.cpu().numpy() - run(x, w, b)) <= bound).all()
 
 
+def precise(got, want, terms, more=0.0):
+    """The root mean square of the error against 64 bits, for sums of `terms` random products.
+    Each 16-deep product rounds the running sum once (to 2^-24 of it), the second accumulator,
+    the final addition and the bias a few times more, independently: sqrt(terms / 16 + 4)
+    roundings, and `more` for what comes with them. A partial product left out, hi lo the least
+    of them, is an error of 2^-18.7 of the sum, the bound under 2^-20 up to 3700 terms."""
+    err = np.sqrt(np.mean((got - want) ** 2)) / np.sqrt(np.mean(want ** 2))
+    bound = (math.sqrt(terms / 16 + 4) + more) * 2.0 ** -24
+    assert err <= bound, (err / 2.0 ** -24, bound / 2.0 ** -24)
+
+
+def conv_exact(x, w, b, dilation=1, stride=1, padding=0, groups=1, positions=None):
+    """Conv1d in 64 bits, x [in][L], w [out][in / groups][k], the first `positions` outputs."""
+    x, w = x.astype(np.float64), w.astype(np.float64)
+    kernel, per = w.shape[2], w.shape[1]
+    n = (x.shape[1] + 2 * padding - (kernel - 1) * dilation - 1) // stride + 1
+    n = n if positions is None else positions
+    x = np.pad(x, ((0, 0), (padding, padding)))
+    y = np.zeros((w.shape[0], n))
+    out = w.shape[0] // groups
+    for g in range(groups):
+        for k in range(kernel):
+            at = x[g * per:(g + 1) * per, k * dilation:k * dilation + (n - 1) * stride + 1:stride]
+            y[g * out:(g + 1) * out] += w[g * out:(g + 1) * out, :, k] @ at
+    return y + b.astype(np.float64)[:, None]
+
+
+@pytest.mark.parametrize("cin,cout,length,kernel,dilation,stride,padding,groups,elu,split", [
+    (1, 65, 1003, 10, 1, 5, 0, 1, False, 0),       # the first feature convolution
+    (40, 130, 611, 3, 1, 2, 0, 1, False, 1 << 20), # a strided window, split
+    (96, 96, 50, 3, 1, 1, 1, 1, True, 1 << 20),    # k3 of an activated input, split
+    (96, 96, 50, 3, 1, 1, 1, 1, True, 0),
+    (64, 40, 333, 16, 1, 8, 4, 1, False, 0),       # a downsampling layer
+    (96, 96, 70, 32, 1, 1, 16, 4, False, 1 << 20), # grouped, an even kernel's first outputs
+    (300, 130, 33, 1, 1, 1, 0, 1, False, 1 << 20), # one tap, split
+    (300, 70, 30, 7, 3, 1, 9, 1, False, 1 << 20),  # seven taps, split, 128 x 32 tiles
+    (520, 300, 190, 7, 1, 1, 3, 1, False, 1 << 20),
+    (40, 24, 70, 7, 1, 1, 3, 1, False, 1 << 20),   # narrow layers, split
+    (70, 64, 90, 7, 9, 1, 27, 1, False, 1 << 20),
+    (33, 129, 8193, 7, 1, 1, 3, 1, False, 0),      # 128 x 64 tiles
+])
+def test_strided_and_split_conv1d_precision(cin, cout, length, kernel, dilation, stride, padding,
+                                            groups, elu, split):
+    rng = np.random.default_rng(cin + cout + length)
+    x = rng.standard_normal((cin, length)).astype(np.float32)
+    per = cin // groups
+    w = (rng.standard_normal((cout, per, kernel)) / math.sqrt(per * kernel)).astype(np.float32)
+    b = (0.1 * rng.standard_normal(cout)).astype(np.float32)
+    positions = (length + 2 * padding - (kernel - 1) * dilation - 1) // stride + 1
+    if kernel % 2 == 0 and padding == kernel // 2:
+        positions = length
+    xin = np.where(x > 0, x, np.expm1(x.astype(np.float64))) if elu else x
+    want = conv_exact(xin, w, b, dilation, stride, padding, groups, positions)
+    y = dev(np.zeros((cout, positions)))
+    ov.op_conv1d_strided(dev(x), w, b, y, dilation, stride, padding, groups, elu, split)
+    # each input of an ELU carries its rounding too
+    precise(y.cpu().numpy(), want, per * kernel, more=1.0 if elu else 0.0)
+
+
+@pytest.mark.parametrize("second", [False, True])
+@pytest.mark.parametrize("channels,length,dilation", [
+    (5, 131, 9), (32, 257, 1), (48, 300, 3), (64, 129, 1), (100, 65, 9), (128, 70, 3),
+    # the wider tiles, which take over where the narrow ones number twice the CUs
+    (40, 32641, 3), (64, 32700, 9), (65, 16321, 1), (96, 16400, 9), (128, 16385, 3)])
+def test_residual_unit_precision(channels, length, dilation, second):
+    """Either product of a fused unit against 64 bits, the other one an exact scaling by powers
+    of two. The Snake, of a small alpha, adds a few roundings and turns the sum by under 1 %."""
+    rng = np.random.default_rng(channels + length)
+    x, y0 = (rng.standard_normal((channels, length)).astype(np.float32) for _ in range(2))
+    alpha = (0.002 * np.exp(0.3 * rng.standard_normal(channels))).astype(np.float32)
+    b1, b2 = (0.1 * rng.standard_normal((2, channels))).astype(np.float32)
+    scaling = np.diag(2.0 ** rng.integers(-2, 3, channels)).astype(np.float32)
+    if second:
+        w1 = np.zeros((channels, channels, 7), np.float32)
+        w1[:, :, 3] = scaling
+        w2 = rng.standard_normal((channels, channels)) / math.sqrt(channels)
+    else:
+        w1 = rng.standard_normal((channels, channels, 7)) / math.sqrt(7 * channels)
+        w2 = scaling
+    w1, w2 = w1.astype(np.float32), w2.astype(np.float32)
+    v = conv_exact(x, w1, b1, dilation, padding=3 * dilation)
+    a = alpha.astype(np.float64)[:, None]
+    v = v + np.sin(a * v) ** 2 / (a + 1e-9)
+    want = conv_exact(v, w2[:, :, None], b2) + y0
+    y = dev(y0)
+    ov.op_residual_unit(dev(x), w1, b1, dev(alpha), w2, b2, y, dilation)
+    precise(y.cpu().numpy(), want, channels * (1 if second else 7), more=2.0)
+
+
 @pytest.mark.parametrize("channels,frames", [(32, 5), (64, 11), (128, 23), (192, 43), (256, 3)])
 def test_fused_residual_units_match_oracle(channels, frames):
-    """Decoders whose blocks' units run fused at every tile (16 to 128 channels, ragged ones
-    too), next to 256 channels that do not."""
+    """Decoders whose blocks' units run fused (16 to 128 channels, ragged ones too; the narrower
+    tiles, at signals this short), next to 256 channels that do not."""
     cfg = dict(TINY, channels=channels * 2, ratios=[5, 2])
     codes = np.random.default_rng(frames).integers(0, 16, size=(3, frames)).astype(np.int32)
     close(ov.Codec.synthetic(cfg, 31).decode(codes), oracle.Codec(cfg, 31).decode(codes),

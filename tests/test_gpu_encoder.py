@@ -76,6 +76,56 @@ def test_attention_shapes_match_oracle(width, heads, frames):
     compare(got, oracle.Encoder(cfg, 21).encode(x))
 
 
+@pytest.mark.parametrize("heads,dim,steps", [
+    (3, 4, 30), (2, 64, 33), (2, 80, 261), (1, 64, 1045), (1, 320, 70), (1, 257, 32)])
+def test_attention_precision(heads, dim, steps):
+    """The attention against 64 bits, scores of unit variance. A score's roundings (dim / 16
+    products and a few more), each of 2^-24 of it, and the exponential's two are the relative
+    error of an independent probability; the context's sum adds steps / 16 roundings. A partial
+    product of the scores or the context left out is an error of 2^-18.7 or more."""
+    import torch
+    rng = np.random.default_rng(dim + steps)
+    q, k, v = (rng.standard_normal((heads, dim, steps)).astype(np.float32) for _ in range(3))
+    scale = dim ** -0.5
+    scores = np.einsum("hdt,hds->hts", q.astype(np.float64), k.astype(np.float64))
+    scores *= np.float64(np.float32(scale))
+    p = np.exp(scores - scores.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    want = np.einsum("hds,hts->hdt", v.astype(np.float64), p)
+    out = torch.zeros((heads, dim, steps), device="cuda")
+    ov.op_head_attention(*(torch.from_numpy(a).cuda() for a in (q, k, v)), out, scale)
+    err = out.cpu().numpy() - want
+    rel = np.sqrt((err ** 2).mean() / (want ** 2).mean()) * 2.0 ** 24
+    assert rel <= np.sqrt(dim / 16 + 8) + np.sqrt(steps / 16), rel
+
+
+@pytest.mark.parametrize("hidden,frames,dim,entries", [
+    (36224, 3, 64, 20),   # the residual fills the work-group's LDS
+    (36225, 3, 64, 20),   # and no longer fits it
+    (40000, 2, 5, 1100),
+    (17792, 257, 64, 4),  # two frames' residuals fill it
+    (17793, 258, 64, 4)])
+def test_quantizer_residual_in_memory(hidden, frames, dim, entries):
+    """The quantizer at the largest residuals that stay in LDS, and past them, against 64 bits."""
+    import torch
+    stages = 3
+    rng = np.random.default_rng(hidden)
+    x = rng.standard_normal((hidden, frames)).astype(np.float32)
+    project = (rng.standard_normal((stages, dim, hidden)) / np.sqrt(hidden)).astype(np.float32)
+    bias = rng.standard_normal((stages, dim)).astype(np.float32)
+    embed = rng.standard_normal((stages, entries, dim)).astype(np.float32)
+    table = rng.standard_normal((stages, entries, hidden)).astype(np.float32)
+    codes = torch.zeros((stages, frames), dtype=torch.int32, device="cuda")
+    ov.op_quantize(torch.from_numpy(x).cuda(), project, bias, embed, table, codes)
+    r, want = x.T.astype(np.float64), []
+    for s in range(stages):
+        p = r @ project[s].T.astype(np.float64) + bias[s]
+        e = embed[s].astype(np.float64)
+        want.append((((p[:, None] - e) ** 2).sum(-1)).argmin(-1))
+        r = r - table[s][want[-1]]
+    np.testing.assert_array_equal(codes.cpu().numpy(), np.array(want))
+
+
 @pytest.mark.parametrize("frames,dim,size", [
     (9, 70, 1500),   # dims and entries past one round of the lanes and threads
     (300, 8, 1024),  # two frames per work-group

@@ -54,7 +54,7 @@ void LaunchPackConvWeights(const float* w, int lead, int taps, int cin, int cout
 // launch is a residual unit of up to kConvFusedChannels channels: v passes
 // through the Snake of alpha_mid and the one-tap convolution w2, bias2 before
 // the residual (x is then neither y nor y_act). Either
-// output may be null; bias may be null (zero); residual may be y.
+// output may be null; bias may be null (zero); residual may be y (phases have none).
 // `batches` independent convolutions of the same shape run in one launch, the
 // pointers of batch b advanced by b times their batch strides, the weights by
 // one lead (a grouped convolution).

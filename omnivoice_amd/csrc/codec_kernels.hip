@@ -50,20 +50,96 @@ __device__ __forceinline__ float Gelu(float v) {
 __device__ __forceinline__ float Elu(float v) { return v > 0.0F ? v : expm1f(v); }
 
 // The epilogue of one output: bias, pre-activation, residual accumulation,
-// the stores.
-__device__ __forceinline__ void Finish(const ConvParams& p, const float* bias,
-                                       const float* residual, float* y, float* y_act, int co,
-                                       size_t at, float v) {
-  if (bias != nullptr)
-    v += bias[co];
+// the stores. What it reads is given, loaded before the sum is known.
+struct Extras {
+  float bias, residual, alpha;
+};
+__device__ __forceinline__ Extras LoadExtras(const ConvParams& p, const float* bias,
+                                             const float* residual, const float* y_act, int co,
+                                             size_t at) {
+  return {bias != nullptr ? bias[co] : 0.0F, residual != nullptr ? residual[at] : 0.0F,
+          y_act != nullptr && p.out_act == kActSnake ? p.alpha_out[co] : 0.0F};
+}
+__device__ __forceinline__ void Finish(const ConvParams& p, const Extras& x, float* y,
+                                       float* y_act, size_t at, float v) {
+  v += x.bias;
   if (p.pre_act == kActGelu)
     v = Gelu(v);
-  if (residual != nullptr)
-    v += residual[at];
+  v += x.residual;
   if (y != nullptr)
     y[at] = v;
   if (y_act != nullptr)
-    y_act[at] = p.out_act == kActElu ? Elu(v) : Snake(v, p.alpha_out[co], SnakeInverse(p.alpha_out[co]));
+    y_act[at] = p.out_act == kActElu ? Elu(v) : Snake(v, x.alpha, SnakeInverse(x.alpha));
+}
+
+// Weight (tap k, input j, output co) of a lead of packed weights: its parts'
+// sum, exactly.
+__device__ __forceinline__ float PackedWeight(const ConvUnit* w, int rows, int taps, int cin,
+                                              int lead, int k, int j, int co) {
+  const int pad = ConvPad(taps), chunks = (cin + pad - 1) / pad;
+  const size_t step =
+      ((static_cast<size_t>(lead) * chunks + j / pad) * taps + k) * (pad / 16) + j % pad / 16;
+  const auto* at = reinterpret_cast<const std::uint16_t*>(
+                       w + (step * 6 + j % 16 / 8) * rows + co) + j % 8;
+  float part[3];
+#pragma unroll
+  for (int s = 0; s < 3; ++s)
+    part[s] = __builtin_bit_cast(
+        float, static_cast<unsigned>(at[static_cast<size_t>(16 * s) * rows]) << 16);
+  return __builtin_isfinite(part[0]) ? part[0] + (part[1] + part[2]) : part[0];
+}
+
+// One convolution sum (before its bias) from the operands themselves, in
+// double. For sums whose split products are infinite or NaN: an operand is,
+// or is a finite input too large for its first part (split.hpp), or the sum
+// overflows. Such sums are rare, and end at the first NaN.
+__device__ __forceinline__ float WideSum(const ConvParams& p, int batch, int phase, int co, int m) {
+  const float* x = p.x + batch * p.x_batch;
+  double sum = 0.0;
+#pragma unroll 1
+  for (int k = 0; k < p.taps; ++k)
+#pragma unroll 1
+    for (int j = 0; j < p.cin && sum == sum; ++j) {
+      int c = j, t = m + p.first[phase] + k * p.dilation;
+      if (p.view_kernel != 0) {
+        c = j / p.view_kernel;
+        t = m * p.view_stride + p.first[0] + j % p.view_kernel;
+      }
+      float v = 0.0F;
+      if (t >= 0 && t < p.len_in) {
+        v = x[static_cast<size_t>(c) * p.len_in + t];
+        if (p.alpha_in != nullptr)
+          v = Snake(v, p.alpha_in[c], SnakeInverse(p.alpha_in[c]));
+        if (p.in_act == kActElu)
+          v = Elu(v);
+      }
+      sum += static_cast<double>(v) * PackedWeight(p.w, p.w_rows, p.taps, p.cin,
+                                                   p.phases > 1 ? phase : batch, k, j, co);
+    }
+  return static_cast<float>(sum);
+}
+
+// The same of a residual unit's second convolution.
+__device__ __forceinline__ float WideUnitSum(const ConvParams& p, int co, int m) {
+  double sum = 0.0;
+#pragma unroll 1
+  for (int j = 0; j < p.cout && sum == sum; ++j) {
+    const float v = Snake(WideSum(p, 0, 0, j, m) + p.bias[j], p.alpha_mid[j],
+                          SnakeInverse(p.alpha_mid[j]));
+    sum += static_cast<double>(v) * PackedWeight(p.w2, p.w_rows, 1, p.cout, 0, 0, j, co);
+  }
+  return static_cast<float>(sum);
+}
+
+// A kernel's parameters (its only argument), read again: what rare code uses
+// of them needs no scalar registers before it. With those kept from the start
+// of the kernel a launch took 0.2 us longer.
+__device__ __forceinline__ const ConvParams& ParamsAgain() {
+  auto at = reinterpret_cast<std::uintptr_t>(
+      (__attribute__((address_space(4))) const void*)__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(at));
+  return *(const ConvParams*)(reinterpret_cast<
+                              __attribute__((address_space(4))) const ConvParams*>(at));
 }
 
 // Four floats at any 4-byte address.
@@ -333,20 +409,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
   };
 
   // The weights of the wave's 32 rows, one step after the other.
-  const int steps = (c_end - c_begin) * kSteps;
   const size_t step_units = 6 * static_cast<size_t>(p.w_rows);
   const uintx4* w = reinterpret_cast<const uintx4*>(p.w) +
                     (static_cast<size_t>(rest) * ((p.cin + ConvPad(TAPS) - 1) / ConvPad(TAPS)) *
                          (ConvPad(TAPS) / 16 * TAPS) +
                      c_begin * kSteps) * step_units +
                     static_cast<size_t>(half) * p.w_rows + min(co0 + row + l32, p.w_rows - 1);
-  int ahead = 0;  // the next step to load, held at the last one
   auto load = [&](uintx4* a) {
 #pragma unroll
     for (int s = 0; s < 3; ++s)
       a[s] = w[static_cast<size_t>(2 * s) * p.w_rows];
-    if (++ahead < steps)
-      w += step_units;
+    w += step_units;
   };
 
   constexpr int kTurn = NT > 1 ? 2 : 1;  // blocks multiplied in turn
@@ -407,7 +480,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
             for (int n = g * kSlices / kOver; n < (g + 1) * kSlices / kOver; ++n)
               slice(n, chunk + 1, 1 - buf, d);
           });
-      if (t + kTurn == NT)
+      if (t + kTurn == NT && (more || step + kAhead < kSteps))
         load(a[step % kAhead]);
     }
     if (more) {
@@ -443,10 +516,13 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     for (int t = 0; t < NT; ++t) {
       const int m = m0 + col + 32 * t + l32;
 #pragma unroll
+      for (int r = 0; r < 16; ++r)
+        main[t][r] += low[t][r];
+#pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int co = co0 + row + 8 * (r >> 2) + 4 * half + (r & 3);
         if (m < p.positions && co < p.cout)
-          part[static_cast<size_t>(co) * p.positions + m] = Join(main[t][r], low[t][r]);
+          part[static_cast<size_t>(co) * p.positions + m] = main[t][r];
       }
     }
     return;
@@ -479,7 +555,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
         float v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          v[r] = Snake(Join(main[t][4 * g + r], low[t][4 * g + r]) + bias4[r], alpha4[r],
+          v[r] = Snake((main[t][4 * g + r] + low[t][4 * g + r]) + bias4[r], alpha4[r],
                        inverse4[r]);
           v[r] = row + 8 * g + 4 * half + r < p.cout ? v[r] : 0.0F;
         }
@@ -535,7 +611,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
   // far as the compiler knows.
   float* y = p.y != nullptr ? p.y + batch * p.y_batch : nullptr;
   float* y_act = p.y_act != nullptr ? p.y_act + batch * p.y_batch : nullptr;
-  const float* residual = p.residual != nullptr ? p.residual + batch * p.y_batch : nullptr;
+  const float* residual =
+      !UP && p.residual != nullptr ? p.residual + batch * p.y_batch : nullptr;
   constexpr int kRuns = BN * S / 4;      // per row
   constexpr int kStride = kT / kRuns;    // rows between a thread's runs
   constexpr int kPer = kOutRows / kStride / 4;
@@ -547,7 +624,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     float bias[4], alpha[4];
     floatx4 residual[4];
   };
-  auto gather = [&](int first) {
+  auto gather = [&](int first) __attribute__((always_inline)) {
     Runs v;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -578,28 +655,46 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
 #pragma unroll
         for (int r = 0; r < 8; ++r)
           out[(8 * (r >> 2) + 4 * half + (r & 3)) * kRowFloats + (32 * t + l32) * S + phase] =
-              Join(main[t][r0 / 2 + r], low[t][r0 / 2 + r]);
+              main[t][r0 / 2 + r] + low[t][r0 / 2 + r];
     } else if (row >= r0 && row < r0 + kOutRows) {
 #pragma unroll
       for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
           out[(row - r0 + 8 * (r >> 2) + 4 * half + (r & 3)) * kRowFloats + col + 32 * t + l32] =
-              Join(main[t][r], low[t][r]);
+              main[t][r] + low[t][r];
     }
     __syncthreads();
+    bool wide = false;
+    // Four runs, and whether all of them are finite.
+    auto fours = [&](int q, floatx4* v) __attribute__((always_inline)) {
+      floatx4 zero = {0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[i] = *reinterpret_cast<const floatx4*>(
+            out + (mine - r0 + (4 * q + i) * kStride) * kRowFloats + tid % kRuns * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          zero[e] = fmaf(v[i][e], 0.0F, zero[e]);
+      }
+      return (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.0F;
+    };
 #pragma unroll 1
     for (int q = 0; q < kPer; ++q) {
       const Runs cur = next;
       if (q + 1 < kPer)
         next = gather(mine + 4 * (q + 1) * kStride);
+      floatx4 sums[4];
+      const bool finite = fours(q, sums);
+      wide |= !finite;
+      if (!UP && __builtin_expect(!finite, 0))  // y may be the residual
+        continue;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int local = mine + (4 * q + i) * kStride;
         if (co0 + local >= p.cout || n <= 0)
           continue;
-        floatx4 v = *reinterpret_cast<const floatx4*>(out + (local - r0) * kRowFloats +
-                                                      tid % kRuns * 4);
+        floatx4 v = sums[i];
         const size_t to = static_cast<size_t>(co0 + local) * p.len_out + at0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -625,6 +720,28 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
           else
             for (int e = 0; e < n; ++e)
               y_act[to + e] = v[e];
+        }
+      }
+    }
+    // The sums that are not finite are formed again, and their fours finished.
+    if (__builtin_expect(wide, 0)) {
+      const ConvParams& wp = ParamsAgain();
+#pragma unroll 1
+      for (int q = 0; q < kPer; ++q) {
+        floatx4 sums[4];
+        if (fours(q, sums))
+          continue;
+#pragma unroll 1
+        for (int k = 0; k < 16; ++k) {
+          const int local = mine + (4 * q + k / 4) * kStride, t = at0 + k % 4;
+          const int co = co0 + local;
+          if (co >= wp.cout || k % 4 >= n)
+            continue;
+          float v = out[(local - r0) * kRowFloats + tid % kRuns * 4 + k % 4];
+          if (!__builtin_isfinite(v))
+            v = FUSED ? WideUnitSum(wp, co, t) : WideSum(wp, batch, UP ? t % S : 0, co, t / S);
+          const size_t at = static_cast<size_t>(co) * wp.len_out + t;
+          Finish(wp, LoadExtras(wp, bias, residual, y_act, co, at), y, y_act, at, v);
         }
       }
     }
@@ -656,7 +773,7 @@ __global__ __launch_bounds__(kThreads) void PackConvWeightsKernel(const float* w
       v[i] = c < cin && o < cout ? w[((ld * taps + tap) * cin + c) * cout + o] : 0.0F;
     }
     uintx4 part[3];
-    Split8(v, part);
+    Split8<true>(v, part);
     uintx4* to = out + (at * (groups / 2) + (g >> 1)) * 6 * rows + (g & 1) * static_cast<size_t>(rows) + o;
 #pragma unroll
     for (int s = 0; s < 3; ++s)
@@ -675,18 +792,21 @@ __global__ __launch_bounds__(kThreads) void SplitReduceKernel(ConvParams p) {
     const size_t within = e % per;
     const int co = static_cast<int>(within / p.positions);
     const int m = static_cast<int>(within % p.positions);
-    const float* part = p.partial + static_cast<size_t>(rest) * p.splits * per + within;
-    float v = 0.0F;
-#pragma unroll 8
-    for (int s = 0; s < p.splits; ++s)
-      v += part[static_cast<size_t>(s) * per];
     const int phase = rest % p.phases, batch = rest / p.phases;
     const float* bias = p.bias != nullptr ? p.bias + batch * p.b_batch : nullptr;
     float* y = p.y != nullptr ? p.y + batch * p.y_batch : nullptr;
     float* y_act = p.y_act != nullptr ? p.y_act + batch * p.y_batch : nullptr;
     const float* residual = p.residual != nullptr ? p.residual + batch * p.y_batch : nullptr;
-    const size_t t = static_cast<size_t>(m) * p.phases + phase;
-    Finish(p, bias, residual, y, y_act, co, static_cast<size_t>(co) * p.len_out + t, v);
+    const size_t at = static_cast<size_t>(co) * p.len_out + static_cast<size_t>(m) * p.phases + phase;
+    const Extras extras = LoadExtras(p, bias, residual, y_act, co, at);
+    const float* part = p.partial + static_cast<size_t>(rest) * p.splits * per + within;
+    float v = 0.0F;
+#pragma unroll 8
+    for (int s = 0; s < p.splits; ++s)
+      v += part[static_cast<size_t>(s) * per];
+    if (__builtin_expect(!__builtin_isfinite(v), 0))
+      v = WideSum(ParamsAgain(), batch, phase, co, m);
+    Finish(p, extras, y, y_act, at, v);
   }
 }
 
@@ -922,7 +1042,8 @@ void LaunchConv(const ConvParams& params, hipStream_t stream) {
           "conv: empty shape");
   Require(p.taps == 1 || p.taps == 2 || p.taps == 7, "conv: 1, 2 or 7 taps");
   Require(p.phases >= 1 && p.phases <= kConvMaxPhases, "conv: 1 to 8 phases");
-  Require(p.phases == 1 || (p.taps == 2 && p.batches == 1), "conv: phases have two taps");
+  Require(p.phases == 1 || (p.taps == 2 && p.batches == 1 && p.residual == nullptr),
+          "conv: phases have two taps and no residual");
   for (int i = 1; i < p.phases; ++i)
     Require(p.first[i] - p.first[0] == 0 || p.first[i] - p.first[0] == 1,
             "conv: the phases' windows differ by one position at most");

@@ -199,6 +199,10 @@ __global__ __launch_bounds__(kThreads) void ColumnNormKernel(ColumnNormParams p)
 constexpr int kAttentionTile = 32;   // queries per work-group, keys per tile
 constexpr int kAttentionDims = 64;   // output dims per work-group
 constexpr int kAttentionThreads = 512;
+// What a probability of one counts as until the sums are divided: an exact
+// factor that keeps the weighted sum of up to 2^16 values from overflowing
+// where their mean does not.
+constexpr float kShare = 0x1p-16F;
 // 16-byte vectors of one tile of q or k and of v.
 __host__ __device__ constexpr int QkVectors(int head_dim) { return (head_dim + 15) / 16 * 192; }
 __host__ __device__ constexpr int ValueVectors(int head_dim) {
@@ -238,7 +242,7 @@ __global__ __launch_bounds__(kThreads) void PackHeadsKernel(HeadAttentionParams 
         v[i] = 0.0F;
     }
     uintx4 part[3];
-    Split8(v, part);
+    Split8<true>(v, part);
 #pragma unroll
     for (int k = 0; k < 3; ++k)
       to[((e >> 6) * 3 + k) * 64 + lane] = part[k];
@@ -349,7 +353,8 @@ __global__ __launch_bounds__(kAttentionThreads) void HeadAttentionKernel(HeadAtt
     double part = 0.0;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < T ? expf((s[r] - top) * p.scale) : 0.0F;
+      s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < T ? expf((s[r] - top) * p.scale) * kShare
+                                                        : 0.0F;
       part += s[r];
     }
     sum = sum * keep + (part + __shfl_xor(part, 32));
@@ -363,7 +368,7 @@ __global__ __launch_bounds__(kAttentionThreads) void HeadAttentionKernel(HeadAtt
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
       uintx4 pf[3];
-      Split8(s + 8 * j, pf);
+      Split8<false>(s + 8 * j, pf);
 #pragma unroll
       for (int n = 0; n < 2; ++n) {
         corr[n] = MfmaBf16(vf[n][j][2], pf[0], corr[n]);

@@ -1,7 +1,8 @@
 // Float32 products on the bf16 matrix cores.
 //
 // A float32 value is the sum of three bf16 parts, each the rounding of what
-// the ones before it leave (hi, mid, lo: 8 + 8 + 8 significant bits), and six
+// the ones before it leave (hi, mid, lo: 8 + 8 + 8 significant bits; see the
+// end of this comment for the largest and the smallest values), and six
 // of the nine products of two such triples are summed in float32: hi hi in
 // one accumulator; hi mid, mid hi, mid mid, hi lo and lo hi in a second one,
 // added at the end. What is left out is below 2^-24 of the product, half a
@@ -9,6 +10,16 @@
 // once where the float32 matrix cores' 2-deep one rounds eight times, so the
 // sum is nearer to the exact one than theirs. At 16 times the rate of
 // v_mfma_f32_32x32x2_f32, six products are 2.7 times its throughput.
+//
+// Finite values of 0x1.FFp127 (3.396e38) and more round to infinity in the
+// first part. Operands that are split once and stored (weights, the
+// attention's heads) hold it to bf16's largest value. A convolution's input
+// is split for every tile, without the three operations more a value; there
+// such a value makes the sum infinite or NaN, and every sum that is not
+// finite is formed again in double, from the values themselves.
+// At the other end bf16's parts stop at 2^-133: an operand is kept to 2^-24
+// of itself, but to no less than 2^-134, which is more below 2^-110. (The
+// matrix cores take and keep bf16's subnormal values.)
 #ifndef OMNIVOICE_AMD_SPLIT_HPP_
 #define OMNIVOICE_AMD_SPLIT_HPP_
 
@@ -34,14 +45,24 @@ __device__ __forceinline__ floatx2 Rest(floatx2 v, unsigned pair) {
                  v[1] - __builtin_bit_cast(float, pair & 0xFFFF0000U)};
 }
 
-// Eight values as the three parts of one 16-byte matrix-core operand. An
-// infinite or NaN value has it in the first part and NaN in the others,
-// which only the second accumulator sees.
+// What the first part is rounded from: finite values of 0x1.FFp127 and more,
+// which would round to infinity, are held to bf16's largest one and have the
+// difference in the other parts.
+__device__ __forceinline__ float First(float v) {
+  constexpr float kMost = 0x1.FEp127F;
+  return fabsf(v) < __builtin_inff() ? fminf(fmaxf(v, -kMost), kMost) : v;
+}
+
+// Eight values as the three parts of one 16-byte matrix-core operand, of any
+// float32 (WIDE) or of those below 0x1.FFp127. An infinite or NaN value has
+// it in the first part and NaN in the others, which only the second
+// accumulator sees.
+template <bool WIDE>
 __device__ __forceinline__ void Split8(const float* v, uintx4* part) {
 #pragma unroll
   for (int q = 0; q < 4; ++q) {
     floatx2 rest{v[2 * q], v[2 * q + 1]};
-    part[0][q] = RoundPair(rest);
+    part[0][q] = RoundPair(WIDE ? floatx2{First(rest[0]), First(rest[1])} : rest);
     rest = Rest(rest, part[0][q]);
     part[1][q] = RoundPair(rest);
     rest = Rest(rest, part[1][q]);

@@ -179,6 +179,96 @@ def test_strided_and_split_conv1d_precision(cin, cout, length, kernel, dilation,
     precise(y.cpu().numpy(), want, per * kernel, more=1.0 if elu else 0.0)
 
 
+def _huge(rng, shape, share=0.03):
+    """Random values, some of them next to the largest float32 (past bf16's largest)."""
+    x = rng.standard_normal(shape).astype(np.float32)
+    top = np.float32(np.finfo(np.float32).max)
+    at = rng.random(shape) < share
+    x[at] = (rng.choice([-1, 1], at.sum()) * top * rng.uniform(0.999, 1.0, at.sum()))
+    return x
+
+
+def _finite_and_close(got, want, size):
+    """Sums formed in double from the operands: one rounding, and those of the bias and what is
+    added after it. Ordinary sums, of under 600 terms here, by the tile edges' bound."""
+    assert np.isfinite(want).all() and np.isfinite(got).all()
+    assert (np.abs(got - want) <= 80 * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.parametrize("cin,cout,length,kernel,stride,groups,split", [
+    (32, 32, 140, 7, 1, 1, 0), (40, 33, 90, 1, 1, 1, 0), (40, 70, 300, 7, 1, 1, 0),
+    (300, 130, 40, 1, 1, 1, 1 << 20), (40, 130, 211, 3, 2, 1, 0), (64, 64, 60, 8, 4, 4, 1 << 20)])
+def test_conv1d_of_the_largest_values(cin, cout, length, kernel, stride, groups, split):
+    """Finite inputs and weights that round to bf16's infinity give finite sums."""
+    rng = np.random.default_rng(cin + cout + kernel)
+    per, padding = cin // groups, (kernel - 1) // 2
+    tiny = 2.0 ** -12
+    b = rng.standard_normal(cout).astype(np.float32)
+    for big_weights in (False, True):
+        x = _huge(rng, (cin, length))
+        w = (tiny * rng.standard_normal((cout, per, kernel))).astype(np.float32)
+        if big_weights:
+            x, w = (tiny * rng.standard_normal(x.shape)).astype(np.float32), _huge(rng, w.shape)
+        want = conv_exact(x, w, b, 1, stride, padding, groups)
+        size = conv_exact(np.abs(x), np.abs(w), np.abs(b), 1, stride, padding, groups)
+        y = dev(np.zeros(want.shape))
+        ov.op_conv1d_strided(dev(x), w, b, y, 1, stride, padding, groups, False, split)
+        _finite_and_close(y.cpu().numpy(), want, size)
+
+
+def test_conv1d_of_the_smallest_values():
+    """Inputs around 2^-118, whose low parts are below bf16's least value 2^-133, against 64
+    bits: each is kept to half of that, beside the tile edges' bound."""
+    rng = np.random.default_rng(7)
+    x = (2.0 ** -118 * rng.standard_normal((40, 300))).astype(np.float32)
+    w = (2.0 ** 20 * rng.standard_normal((33, 40, 7))).astype(np.float32)
+    b = np.zeros(33, np.float32)
+    y = dev(np.zeros((33, 300)))
+    ov.op_conv1d(dev(x), w, b, y)
+    size = conv_exact(np.abs(x), np.abs(w), b, padding=3)
+    kept = np.abs(w).astype(np.float64).sum((1, 2))[:, None] * 2.0 ** -134
+    err = np.abs(y.cpu().numpy() - conv_exact(x, w, b, padding=3))
+    assert (err <= (40 * 7 / 8 + 8) * 2.0 ** -24 * size + kept).all()
+
+
+@pytest.mark.parametrize("cin,cout,length,stride", [(40, 33, 50, 3), (33, 40, 70, 8)])
+def test_conv_transpose1d_of_the_largest_values(cin, cout, length, stride):
+    rng = np.random.default_rng(stride)
+    x, tiny = _huge(rng, (cin, length)), 2.0 ** -12
+    w = (tiny * rng.standard_normal((cin, cout, 2 * stride))).astype(np.float32)
+    b = rng.standard_normal(cout).astype(np.float32)
+    y = dev(np.zeros((cout, length * stride)))
+    ov.op_conv_transpose1d(dev(x), w, b, y, stride)
+
+    def run(x, w, b):
+        full = np.zeros((cout, (length + 2) * stride))
+        for k in range(2 * stride):
+            full[:, k:k + (length - 1) * stride + 1:stride] += w[:, :, k].T @ x
+        pad = (stride + 1) // 2
+        return full[:, pad:pad + length * stride] + b[:, None]
+    x, w, b = (v.astype(np.float64) for v in (x, w, b))
+    _finite_and_close(y.cpu().numpy(), run(x, w, b), run(np.abs(x), np.abs(w), np.abs(b)))
+
+
+@pytest.mark.parametrize("channels,length", [(20, 150), (48, 140), (100, 66), (65, 16321)])
+def test_residual_unit_of_the_largest_values(channels, length):
+    """Inputs, and results of the first convolution, that round to bf16's infinity. Alphas of
+    one: the Snake adds at most one, of nothing to such values."""
+    rng = np.random.default_rng(channels)
+    x = _huge(rng, (channels, length), share=20.0 / (channels * length))
+    w1 = np.zeros((channels, channels, 7), np.float32)
+    w1[:, :, 3] = np.eye(channels)
+    w2 = (2.0 ** -12 * rng.standard_normal((channels, channels))).astype(np.float32)
+    zero = np.zeros(channels, np.float32)
+    y0 = rng.standard_normal((channels, length)).astype(np.float32)
+    v = x.astype(np.float64)
+    v = v + np.where(np.abs(v) < 1e6, np.sin(v) ** 2, 0.0)
+    size = conv_exact(np.abs(v), np.abs(w2)[:, :, None], zero) + np.abs(y0)
+    y = dev(y0)
+    ov.op_residual_unit(dev(x), w1, zero, dev(np.ones(channels)), w2, zero, y)
+    _finite_and_close(y.cpu().numpy(), conv_exact(v, w2[:, :, None], zero) + y0, size)
+
+
 @pytest.mark.parametrize("second", [False, True])
 @pytest.mark.parametrize("channels,length,dilation", [
     (5, 131, 9), (32, 257, 1), (48, 300, 3), (64, 129, 1), (100, 65, 9), (128, 70, 3),

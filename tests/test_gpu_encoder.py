@@ -99,6 +99,28 @@ def test_attention_precision(heads, dim, steps):
     assert rel <= np.sqrt(dim / 16 + 8) + np.sqrt(steps / 16), rel
 
 
+@pytest.mark.parametrize("dim,steps", [(8, 30), (64, 300), (320, 40)])
+def test_attention_of_the_largest_values(dim, steps):
+    """Values, and keys, that round to bf16's infinity; and a mean of values whose sum would
+    overflow."""
+    import torch
+    rng = np.random.default_rng(dim)
+    top = np.float32(np.finfo(np.float32).max)
+    q, k, v = (rng.standard_normal((1, dim, steps)).astype(np.float32) for _ in range(3))
+    v[0, 0], v[0, 1, ::3], v[0, 2, 5] = top, -top, top * np.float32(0.9995)
+    k[0, 3, 7], q[0, 3] = top, np.float32(2.0 ** -100) * q[0, 3]  # the only key, or none
+    out = torch.zeros((1, dim, steps), device="cuda")
+    ov.op_head_attention(*(torch.from_numpy(a).cuda() for a in (q, k, v)), out, 0.25)
+    scores = 0.25 * (q[0].T.astype(np.float64) @ k[0].astype(np.float64))
+    p = np.exp(scores - scores.max(-1, keepdims=True))
+    want = v[0].astype(np.float64) @ (p / p.sum(-1, keepdims=True)).T
+    got = out[0].cpu().numpy().astype(np.float64)
+    # a mean of the largest value alone may exceed it by its roundings
+    assert np.isfinite(got[1:]).all() and (got[0] >= top * (1 - 2.0 ** -18)).all()
+    size = np.abs(v[0]).astype(np.float64) @ (p / p.sum(-1, keepdims=True)).T
+    assert (np.abs(got[1:] - want[1:]) <= 2.0 ** -18 * size[1:]).all()
+
+
 @pytest.mark.parametrize("hidden,frames,dim,entries", [
     (36224, 3, 64, 20),   # the residual fills the work-group's LDS
     (36225, 3, 64, 20),   # and no longer fits it

@@ -107,20 +107,22 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length,
                             int64_t out, int64_t stride, float* y, void* stream,
                             char* error, size_t error_len);
 
-/* A strided, grouped or split convolution for op-level tests: x [in][length]
- * and y [out][positions] in device memory; w [out][in / groups][kernel] and
- * b [out] on the host; ELU on the input when elu is set. One group of 1, 2
+/* A strided, grouped or split convolution for op-level tests: x [in][length],
+ * alpha [in] and y [out][positions] in device memory; w [out][in /
+ * groups][kernel] and b [out] on the host; on the input Snake when alpha is
+ * not NULL (one group only), then ELU when elu is set. One group of 1, 2
  * or 7 taps at stride 1 with padding (kernel - 1) dilation / 2 on each side
  * and as many outputs as inputs runs tap by tap, everything else (dilation
  * 1) through a strided window of the input. `split_floats` is the size of a
  * workspace with which the input channels may be split (0: none).
  * Synchronises `stream`. */
 int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length,
-                          const float* w, const float* b, int64_t out,
-                          int64_t kernel, int64_t dilation, int64_t stride,
-                          int64_t padding, int64_t groups, int elu,
-                          int64_t split_floats, float* y, int64_t positions,
-                          void* stream, char* error, size_t error_len);
+                          const float* alpha, const float* w, const float* b,
+                          int64_t out, int64_t kernel, int64_t dilation,
+                          int64_t stride, int64_t padding, int64_t groups,
+                          int elu, int64_t split_floats, float* y,
+                          int64_t positions, void* stream, char* error,
+                          size_t error_len);
 
 /* A residual unit of up to 128 channels for op-level tests: y += w2
  * snake(w1 x + b1) + b2, w1 [channels][channels][7] at `dilation`, w2

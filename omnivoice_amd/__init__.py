@@ -155,9 +155,9 @@ EXPORTS = {
                                      ctypes.c_int, _ptr, _ptr, _err, _sz]),
     "ovc_op_conv_transpose1d": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr, _i64,
                                                _i64, _ptr, _ptr, _err, _sz]),
-    "ovc_op_conv1d_strided": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _i64, _i64, _i64,
-                                             _i64, _i64, _i64, ctypes.c_int, _i64, _ptr, _i64,
-                                             _ptr, _err, _sz]),
+    "ovc_op_conv1d_strided": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _ptr, _i64, _i64,
+                                             _i64, _i64, _i64, _i64, ctypes.c_int, _i64, _ptr,
+                                             _i64, _ptr, _err, _sz]),
     "ovc_op_residual_unit": (ctypes.c_int, [_ptr, _i64, _i64, _ptr, _ptr, _i64, _ptr, _ptr,
                                             _ptr, _ptr, _ptr, _err, _sz]),
     # the audio encoder (include/omnivoice_codec_mi355x.h)
@@ -761,16 +761,17 @@ def op_conv_transpose1d(x, w, b, y, stride: int, alpha=None, stream=None) -> Non
 
 def op_conv1d_strided(x, w, b, y, dilation: int = 1, stride: int = 1, padding: int = 0,
                       groups: int = 1, elu: bool = False, split_floats: int = 0,
-                      stream=None) -> None:
-    """x [in][L] and y [out][positions]: float32 device tensors; w
+                      alpha=None, stream=None) -> None:
+    """x [in][L], y [out][positions], alpha [in]: float32 device tensors; w
     [out][in / groups][k] and b [out]: host float32 arrays."""
     w = np.ascontiguousarray(w, dtype=np.float32)
     b = np.ascontiguousarray(b, dtype=np.float32)
     err = _buf()
-    _check(lib().ovc_op_conv1d_strided(_dev(x), x.shape[0], x.shape[1], _p(w), _p(b), w.shape[0],
-                                       w.shape[2], dilation, stride, padding, groups, int(elu),
-                                       split_floats, _dev(y), y.shape[1], _stream(stream), err,
-                                       len(err)), err)
+    _check(lib().ovc_op_conv1d_strided(_dev(x), x.shape[0], x.shape[1],
+                                       _dev(alpha) if alpha is not None else None, _p(w), _p(b),
+                                       w.shape[0], w.shape[2], dilation, stride, padding, groups,
+                                       int(elu), split_floats, _dev(y), y.shape[1],
+                                       _stream(stream), err, len(err)), err)
 
 
 def op_residual_unit(x, w1, b1, alpha, w2, b2, y, dilation: int = 1, stream=None) -> None:

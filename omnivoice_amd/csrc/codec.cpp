@@ -660,11 +660,11 @@ int ovc_op_conv_transpose1d(const float* x, int64_t in, int64_t length, const fl
   });
 }
 
-int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length, const float* w,
-                          const float* b, int64_t out, int64_t kernel, int64_t dilation,
-                          int64_t stride, int64_t padding, int64_t groups, int elu,
-                          int64_t split_floats, float* y, int64_t positions, void* stream,
-                          char* error, size_t error_len) {
+int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length, const float* alpha,
+                          const float* w, const float* b, int64_t out, int64_t kernel,
+                          int64_t dilation, int64_t stride, int64_t padding, int64_t groups,
+                          int elu, int64_t split_floats, float* y, int64_t positions,
+                          void* stream, char* error, size_t error_len) {
   return CodecGuard("conv1d_strided: ", error, error_len, [&] {
     ovg::Require(x && w && b && y, "null pointer");
     const int64_t limit = int64_t{1} << 31;
@@ -680,6 +680,7 @@ int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length, const floa
                       (kernel == 1 || kernel == 2 || kernel == 7) &&
                       padding == (kernel - 1) * dilation / 2;
     ovg::Require(taps || dilation == 1, "a strided or grouped convolution is not dilated");
+    ovg::Require(groups == 1 || alpha == nullptr, "a grouped convolution has no Snake");
     const int K = static_cast<int>(kernel), G = static_cast<int>(groups);
     const int I = static_cast<int>(in) / G, O = static_cast<int>(out) / G;
     std::vector<float> layout;
@@ -719,6 +720,7 @@ int ovc_op_conv1d_strided(const float* x, int64_t in, int64_t length, const floa
       p.b_batch = O;
       p.y_batch = static_cast<int64_t>(O) * positions;
     }
+    p.alpha_in = alpha;
     p.in_act = elu ? ovg::kActElu : ovg::kActNone;
     p.partial = split_floats > 0 ? partial.get() : nullptr;
     p.partial_capacity = split_floats;

@@ -373,7 +373,8 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
       const int j = chunk * kChunk + 8 * group[q];
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float alpha = p.alpha_in != nullptr ? p.alpha_in[min(j + i, p.cin - 1)] : 0.0F;
+        const int c = VIEW ? min((j + i) / p.view_kernel, p.channels - 1) : min(j + i, p.cin - 1);
+        const float alpha = p.alpha_in != nullptr ? p.alpha_in[c] : 0.0F;
         float& v = window[d][q][i];
         if (p.alpha_in != nullptr)
           v = Snake(v, alpha, SnakeInverse(alpha));

@@ -179,6 +179,20 @@ def test_strided_and_split_conv1d_precision(cin, cout, length, kernel, dilation,
     precise(y.cpu().numpy(), want, per * kernel, more=1.0 if elu else 0.0)
 
 
+@pytest.mark.parametrize("cin,kernel,stride", [(40, 4, 2), (33, 3, 1), (9, 16, 8)])
+def test_strided_conv1d_of_a_snake(cin, kernel, stride):
+    """Each channel of a strided window by its own alpha."""
+    rng = np.random.default_rng(kernel)
+    x = rng.standard_normal((cin, 203)).astype(np.float32)
+    w = (rng.standard_normal((70, cin, kernel)) / math.sqrt(cin * kernel)).astype(np.float32)
+    b = rng.standard_normal(70).astype(np.float32)
+    alpha = np.exp(rng.standard_normal(cin)).astype(np.float32)
+    want = conv_exact(oracle.snake(x, alpha), w, b, 1, stride, 1)
+    y = dev(np.zeros(want.shape))
+    ov.op_conv1d_strided(dev(x), w, b, y, stride=stride, padding=1, alpha=dev(alpha))
+    precise(y.cpu().numpy(), want, cin * kernel, more=4.0)  # the Snake's roundings on both sides
+
+
 def _huge(rng, shape, share=0.03):
     """Random values, some of them next to the largest float32 (past bf16's largest)."""
     x = rng.standard_normal(shape).astype(np.float32)

@@ -86,7 +86,7 @@ struct ConvParams {
   float* partial;
   std::int64_t partial_capacity;
   // Set by the launcher.
-  int splits, split_chunks, w_rows, rows_first;
+  int splits, split_chunks, w_rows;
 };
 void LaunchConv(const ConvParams& p, hipStream_t stream);
 

@@ -254,23 +254,17 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
   static_assert(!FUSED || 3 * BM / 8 * BN <= kLds, "the second operand's LDS");
   __shared__ uintx4 xs[kLds];
 
-  // Work-group to tile: consecutive tiles stay on one XCD, the positions of a
-  // row block where the weights are the larger operand, the row blocks of a
-  // position tile where the input is, so that the XCDs' caches do not all
-  // hold the larger one.
+  // Work-group to tile: consecutive tiles, the positions of a row block, stay
+  // on one XCD, whose cache then holds few of the weights. (The row blocks of
+  // a position tile first, or that only where the input is the larger operand:
+  // within 2 % at every layer but the linear ones of 768 channels, where rows
+  // first are slower, 27.8 -> 33.2 us to 3072 channels at 500 positions.)
   const int tiles_n = (p.positions + BN - 1) / BN, tiles_m = (p.cout + BM - 1) / BM;
-  int tile = XcdTile(blockIdx.x, gridDim.x), tile_n, tile_m;
-  if (p.rows_first) {
-    tile_m = tile % tiles_m;
-    tile /= tiles_m;
-    tile_n = tile % tiles_n;
-    tile /= tiles_n;
-  } else {
-    tile_n = tile % tiles_n;
-    tile /= tiles_n;
-    tile_m = tile % tiles_m;
-    tile /= tiles_m;
-  }
+  int tile = XcdTile(blockIdx.x, gridDim.x);
+  const int tile_n = tile % tiles_n;
+  tile /= tiles_n;
+  const int tile_m = tile % tiles_m;
+  tile /= tiles_m;
   const int split = tile % p.splits;
   const int batch = tile / p.splits;
   const int chunks = (p.cin + kChunk - 1) / kChunk;

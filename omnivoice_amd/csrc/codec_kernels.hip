@@ -918,12 +918,21 @@ int64_t Tiles(const ConvParams& p, int bm, int bn) {
 // when the input is one chunk, so that two work-groups' windows fit a CU's
 // LDS, else 32 x 128; 64 x 128; about 512 work-groups.
 //
-// Wider layers take 128 x 64, or 128 x 32 while that leaves CUs idle; a split
-// costs a pass of partial sums, so it only has to give each CU one work-group,
-// unless the sums are so long (over 512 channels x 7 taps) that three balance
-// better. Measured at one tap, 768 -> 3072 channels: 500 positions 20.6 us at
-// 384 tiles of 128 x 32, 21.3 at 192 of 128 x 64, 29-30 split in two; 1046
-// positions 39.2 and 34.5 (408 tiles of 128 x 64); 768 -> 768 at 150
+// Wider layers take 128 x 64, or 128 x 32 where that keeps the CUs as busy.
+// One tap: up to three narrow tiles a CU cost as much as one wide one, or less
+// than two (768 -> 3072 channels: 216 wide tiles 25.6 us and 25.4 narrow, 264
+// 36.8 and 35.2, 384 39.7 and 38.6, 408 40.3 and 45.6; 3072 -> 768: 360 128
+// and 126, 390 131 and 154; 512 x 3 taps of a view: 200 59.7 and 53.4, 328
+// 89.3 and 82.5, 392 92.7 and 101). Seven taps, with splits: wide ones once
+// they and their splits number the CUs; without: one narrow tile a CU (512
+// channels: 128 wide tiles 64.8 us and 55.4 narrow, 200 70.6 and 78.2), two
+// where the sum is short (32 channels: 200 11.6 and 10.8, 256 12.2 and 11.9,
+// 300 15.4 and 15.6, 512 17.4 and 19.8).
+//
+// A split costs a pass of partial sums, so it only has to give each CU one
+// work-group, unless the sums are so long (over 512 channels x 7 taps) that
+// three balance better. Measured at one tap: 768 -> 3072 channels x 500 20.6
+// us at 384 tiles of 128 x 32, 29-30 split in two; 768 -> 768 at 150
 // positions 15.0 at 30 tiles, 11.9 and 10.7 split in two and three. At seven
 // taps: 512 channels x 2000 positions 63.6 at 128 tiles of 128 x 64, 43.4,
 // 44.9, 48.0 split in two, four, six; x 200 positions 16.4 (16 tiles, eight
@@ -947,8 +956,10 @@ void DispatchTaps(const ConvParams& params, hipStream_t stream) {
   } else {
     const int64_t tiles = Tiles(p, 128, 64);
     const int most = TAPS == 7 ? 8 : 65535;
-    const bool wide = TAPS == 1 ? tiles >= 400
-                                : tiles * std::min(most, (p.cin + 31) / 32 / 2) >= 256;
+    const int splits = p.partial == nullptr ? 1 : std::min(most, (p.cin + 31) / 32 / 2);
+    const bool wide = TAPS == 1    ? Tiles(p, 128, 32) > 3 * kCus
+                      : splits > 1 ? tiles * splits >= kCus
+                                   : Tiles(p, 128, 32) > (p.cin <= 64 ? 2 : 1) * kCus;
     ChooseSplits(&p, wide ? tiles : Tiles(p, 128, 32), TileChunk(TAPS, wide ? 64 : 32),
                  TAPS == 7 && p.cin > 512 ? 768 : 256, most);
     if (wide)

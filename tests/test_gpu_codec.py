@@ -160,6 +160,11 @@ def conv_exact(x, w, b, dilation=1, stride=1, padding=0, groups=1, positions=Non
     (40, 24, 70, 7, 1, 1, 3, 1, False, 1 << 20),   # narrow layers, split
     (70, 64, 90, 7, 9, 1, 27, 1, False, 1 << 20),
     (33, 129, 8193, 7, 1, 1, 3, 1, False, 0),      # 128 x 64 tiles
+    (32, 129, 8201, 7, 9, 1, 27, 1, False, 0),     # the same, of one chunk
+    (17, 200, 8193, 7, 1, 1, 3, 1, False, 1 << 20),
+    (40, 300, 8129, 1, 1, 1, 0, 1, False, 0),      # one tap: past three narrow tiles a CU
+    (40, 300, 8065, 1, 1, 1, 0, 1, False, 0),      # and not
+    (40, 300, 8129, 3, 1, 2, 1, 1, False, 0),
 ])
 def test_strided_and_split_conv1d_precision(cin, cout, length, kernel, dilation, stride, padding,
                                             groups, elu, split):

@@ -491,7 +491,6 @@ Plan EncoderEngine::MakePlan(int64_t length) const {
 
 void EncoderEngine::Reserve(const Plan& p) {
   const int64_t W = W_, T = p.steps, F = p.frames;
-  // cols: the largest convolution's channels x taps x positions, a bound only.
   int64_t feat = 0, cols = 0;
   int64_t in = 1, len = p.resampled + 2 * kWavePad;
   for (int i = 0; i < cfg_.feature_layers; ++i) {
@@ -511,6 +510,9 @@ void EncoderEngine::Reserve(const Plan& p) {
     dac = std::max(dac, ch * cur);
   }
   cols = std::max(cols, 3 * ch * F);
+  // cols (the largest convolution's channels x taps x positions) and scores
+  // size no buffer; they bound the lengths that are accepted. The attention's
+  // operands are indexed in 64 bits and need no bound of their own.
   const int64_t scores = cfg_.heads * T * T;
   const int64_t hid = std::max<int64_t>(in, W) * T;
   const int64_t limit = int64_t{1} << 31;
@@ -542,7 +544,8 @@ void EncoderEngine::Reserve(const Plan& p) {
   grow(ya_, dac);
   grow(joint_, H_ * F);
   grow(emb_, H_ * F);
-  grow(resid_, H_ * F);
+  grow(resid_, static_cast<int64_t>(RvqResidualElements(static_cast<int>(cfg_.codebook_dim), H_,
+                                                        static_cast<int>(F))));
   grow(codes_, cfg_.codebooks * F);
 }
 
@@ -1152,7 +1155,7 @@ int ovc_op_quantize(const float* x, int64_t hidden, int64_t frames, const float*
     ovg::DeviceBuffer<ovg::RvqStage> device;
     ovg::Upload(device, list);
     ovg::DeviceBuffer<float> residual;
-    residual.Reserve(static_cast<std::size_t>(hidden * frames));
+    residual.Reserve(ovg::RvqResidualElements(D, H, F));
     auto s = static_cast<hipStream_t>(stream);
     ovg::LaunchRvqEncode({x, device.get(), residual.get(), codes, static_cast<int>(stages), D, E,
                           H, F},

@@ -80,10 +80,12 @@ struct RvqStage {
 struct RvqEncodeParams {
   const float* x;         // [hidden][frames]
   const RvqStage* stage;  // [stages], device memory
-  float* residual;        // [frames][hidden], workspace
+  float* residual;        // workspace of RvqResidualElements(...)
   std::int32_t* codes;    // [stages][frames]
   int stages, dim, entries, hidden, frames;
 };
+// Elements of `residual`: none where it stays in a work-group's LDS.
+std::size_t RvqResidualElements(int dim, int hidden, int frames);
 void LaunchRvqEncode(const RvqEncodeParams& p, hipStream_t stream);
 
 }  // namespace ovg

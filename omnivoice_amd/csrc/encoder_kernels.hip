@@ -670,11 +670,18 @@ void LaunchPickFrames(const double* sum, int channels, int positions, int stride
            scale, y);
 }
 
+std::size_t RvqResidualElements(int dim, int hidden, int frames) {
+  return RvqLdsBytes(1, dim, hidden) <= kRvqLdsLimit ? 0
+                                                     : static_cast<std::size_t>(hidden) * frames;
+}
+
 void LaunchRvqEncode(const RvqEncodeParams& p, hipStream_t stream) {
-  Require(p.x && p.stage && p.residual && p.codes, "quantizer: null pointer");
+  Require(p.x && p.stage && p.codes, "quantizer: null pointer");
   Require(p.dim >= 1 && p.dim <= kRvqMaxDim && p.entries >= 1 && p.hidden >= 1 &&
               p.frames >= 1 && p.stages >= 1,
           "quantizer: bad shape");
+  Require(p.residual != nullptr || RvqResidualElements(p.dim, p.hidden, p.frames) == 0,
+          "quantizer: no workspace");
   auto launch = [&](auto kernel, int frames, std::uint64_t bytes) {
     Dispatch(kernel, dim3((p.frames + frames - 1) / frames), dim3(kRvqThreads),
              static_cast<std::uint32_t>(bytes), stream, true, true, p);

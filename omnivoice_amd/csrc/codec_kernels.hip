@@ -131,17 +131,6 @@ __device__ __forceinline__ float WideUnitSum(const ConvParams& p, int co, int m)
   return static_cast<float>(sum);
 }
 
-// A kernel's parameters (its only argument), read again: what rare code uses
-// of them needs no scalar registers before it. With those kept from the start
-// of the kernel a launch took 0.2 us longer.
-__device__ __forceinline__ const ConvParams& ParamsAgain() {
-  auto at = reinterpret_cast<std::uintptr_t>(
-      (__attribute__((address_space(4))) const void*)__builtin_amdgcn_kernarg_segment_ptr());
-  asm volatile("" : "+s"(at));
-  return *(const ConvParams*)(reinterpret_cast<
-                              __attribute__((address_space(4))) const ConvParams*>(at));
-}
-
 // Four floats at any 4-byte address.
 typedef float Unaligned4 __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -720,7 +709,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     }
     // The sums that are not finite are formed again, and their fours finished.
     if (__builtin_expect(wide, 0)) {
-      const ConvParams& wp = ParamsAgain();
+      const ConvParams& wp = ParamsAgain<ConvParams>();
 #pragma unroll 1
       for (int q = 0; q < kPer; ++q) {
         floatx4 sums[4];
@@ -800,7 +789,7 @@ __global__ __launch_bounds__(kThreads) void SplitReduceKernel(ConvParams p) {
     for (int s = 0; s < p.splits; ++s)
       v += part[static_cast<size_t>(s) * per];
     if (__builtin_expect(!__builtin_isfinite(v), 0))
-      v = WideSum(ParamsAgain(), batch, phase, co, m);
+      v = WideSum(ParamsAgain<ConvParams>(), batch, phase, co, m);
     Finish(p, extras, y, y_act, at, v);
   }
 }

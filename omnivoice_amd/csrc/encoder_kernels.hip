@@ -199,10 +199,6 @@ __global__ __launch_bounds__(kThreads) void ColumnNormKernel(ColumnNormParams p)
 constexpr int kAttentionTile = 32;   // queries per work-group, keys per tile
 constexpr int kAttentionDims = 64;   // output dims per work-group
 constexpr int kAttentionThreads = 512;
-// What a probability of one counts as until the sums are divided: an exact
-// factor that keeps the weighted sum of up to 2^16 values from overflowing
-// where their mean does not.
-constexpr float kShare = 0x1p-16F;
 // 16-byte vectors of one tile of q or k and of v.
 __host__ __device__ constexpr int QkVectors(int head_dim) { return (head_dim + 15) / 16 * 192; }
 __host__ __device__ constexpr int ValueVectors(int head_dim) {
@@ -247,6 +243,31 @@ __global__ __launch_bounds__(kThreads) void PackHeadsKernel(HeadAttentionParams 
     for (int k = 0; k < 3; ++k)
       to[((e >> 6) * 3 + k) * 64 + lane] = part[k];
   }
+}
+
+// One output in double, for sums that are not finite: the sum of values next
+// to the largest overflows where their mean does not. Ends at the first NaN.
+__device__ __forceinline__ float WideContext(const HeadAttentionParams& p, int head, int d, int t) {
+  const size_t T = p.steps, at = static_cast<size_t>(head) * p.head_dim * T;
+  const auto score = [&](int s) {
+    double sum = 0.0;
+#pragma unroll 1
+    for (int e = 0; e < p.head_dim; ++e)
+      sum += static_cast<double>(p.q[at + e * T + t]) * p.k[at + e * T + s];
+    return sum * p.scale;
+  };
+  double peak = -DBL_MAX, sum = 0.0, out = 0.0;
+#pragma unroll 1
+  for (int s = 0; s < p.steps; ++s) {
+    const double v = score(s), top = v > peak || v != v ? v : peak;
+    const double keep = exp(peak - top), share = exp(v - top);
+    sum = sum * keep + share;
+    out = out * keep + share * p.v[at + d * T + s];
+    peak = top;
+    if (out != out)
+      break;
+  }
+  return static_cast<float>(out / sum);
 }
 
 // A work-group owns one head's 32 queries (and 64 of the head's dims; wider
@@ -353,8 +374,7 @@ __global__ __launch_bounds__(kAttentionThreads) void HeadAttentionKernel(HeadAtt
     double part = 0.0;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < T ? expf((s[r] - top) * p.scale) * kShare
-                                                        : 0.0F;
+      s[r] = k0 + 8 * (r >> 2) + 4 * half + (r & 3) < T ? expf((s[r] - top) * p.scale) : 0.0F;
       part += s[r];
     }
     sum = sum * keep + (part + __shfl_xor(part, 32));
@@ -410,8 +430,12 @@ __global__ __launch_bounds__(kAttentionThreads) void HeadAttentionKernel(HeadAtt
 #pragma unroll
     for (int w = 0; w < kWaves; ++w)
       o += merged[w][d][q] * keep[w];
-    if (q0 + q < T && slab + d < hd)
-      p.out[(static_cast<size_t>(head) * hd + slab + d) * T + q0 + q] = o * inv;
+    o *= inv;
+    if (q0 + q < T && slab + d < hd) {
+      if (__builtin_expect(!__builtin_isfinite(o), 0))
+        o = WideContext(ParamsAgain<HeadAttentionParams>(), head, slab + d, q0 + q);
+      p.out[(static_cast<size_t>(head) * hd + slab + d) * T + q0 + q] = o;
+    }
   }
 }
 

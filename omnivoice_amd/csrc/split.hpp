@@ -15,8 +15,9 @@
 // first part. Operands that are split once and stored (weights, the
 // attention's heads) hold it to bf16's largest value. A convolution's input
 // is split for every tile, without the three operations more a value; there
-// such a value makes the sum infinite or NaN, and every sum that is not
-// finite is formed again in double, from the values themselves.
+// such a value makes the sum infinite or NaN. Every sum that is not finite,
+// for this reason or another, is formed again in double, from the values
+// themselves.
 // At the other end bf16's parts stop at 2^-133: an operand is kept to 2^-24
 // of itself, but to no less than 2^-134, which is more below 2^-110. (The
 // matrix cores take and keep bf16's subnormal values.)
@@ -80,6 +81,18 @@ __device__ __forceinline__ floatx16 MfmaBf16(uintx4 a, uintx4 b, floatx16 c) {
 // NaN (the second is NaN wherever an operand was infinite).
 __device__ __forceinline__ float Join(float main, float rest) {
   return __builtin_isfinite(main) ? main + rest : main;
+}
+
+// A kernel's parameters (its only argument), read again: what the rare code
+// for sums that are not finite uses of them needs no scalar registers before
+// it. With those kept from a kernel's start its launches took 0.2 us longer.
+template <typename Params>
+__device__ __forceinline__ const Params& ParamsAgain() {
+  using Kernarg = __attribute__((address_space(4))) const Params;
+  auto at = reinterpret_cast<std::uintptr_t>(
+      (__attribute__((address_space(4))) const void*)__builtin_amdgcn_kernarg_segment_ptr());
+  asm volatile("" : "+s"(at));
+  return *(const Params*)reinterpret_cast<Kernarg*>(at);
 }
 
 }  // namespace ovg

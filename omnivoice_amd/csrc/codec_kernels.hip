@@ -76,11 +76,13 @@ __device__ __forceinline__ void Finish(const ConvParams& p, const Extras& x, flo
 // sum, exactly.
 __device__ __forceinline__ float PackedWeight(const ConvUnit* w, int rows, int taps, int cin,
                                               int lead, int k, int j, int co) {
-  const int pad = ConvPad(taps), chunks = (cin + pad - 1) / pad;
-  const size_t step =
-      ((static_cast<size_t>(lead) * chunks + j / pad) * taps + k) * (pad / 16) + j % pad / 16;
+  const int log2 = taps == 1 ? 7 : 5;  // of ConvPad(taps)
+  static_assert(ConvPad(1) == 128 && ConvPad(7) == 32, "padding");
+  const int chunks = ((cin - 1) >> log2) + 1, steps = 1 << (log2 - 4);  // of 16, per chunk
+  const int step =
+      ((lead * chunks + (j >> log2)) * taps + k) * steps + ((j >> 4) & (steps - 1));
   const auto* at = reinterpret_cast<const std::uint16_t*>(
-                       w + (step * 6 + j % 16 / 8) * rows + co) + j % 8;
+                       w + (static_cast<size_t>(step) * 6 + (j >> 3 & 1)) * rows + co) + (j & 7);
   float part[3];
 #pragma unroll
   for (int s = 0; s < 3; ++s)
@@ -92,30 +94,51 @@ __device__ __forceinline__ float PackedWeight(const ConvUnit* w, int rows, int t
 // One convolution sum (before its bias) from the operands themselves, in
 // double. For sums whose split products are infinite or NaN: an operand is,
 // or is a finite input too large for its first part (split.hpp), or the sum
-// overflows. Such sums are rare, and end at the first NaN.
+// overflows. Such sums are rare, or many where a NaN has spread: one among
+// the inputs is looked for first (an encode of 10 s with one in it: 98 ms
+// without, now 18; 4.5 of finite samples).
 __device__ __forceinline__ float WideSum(const ConvParams& p, int batch, int phase, int co, int m) {
   const float* x = p.x + batch * p.x_batch;
+  const bool view = p.view_kernel != 0;
+  const int channels = view ? p.channels : p.cin, taps = view ? p.view_kernel : p.taps;
+  const int t0 = m * (view ? p.view_stride : 1) + p.first[phase], dilation = view ? 1 : p.dilation;
+#pragma unroll 1
+  for (int k = 0; k < taps; ++k) {
+    const int t = t0 + k * dilation;
+    if (t < 0 || t >= p.len_in)
+      continue;
+#pragma unroll 1
+    for (int c0 = 0; c0 < channels; c0 += 8) {
+      float zero = 0.0F;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const float v = x[static_cast<size_t>(min(c0 + i, channels - 1)) * p.len_in + t];
+        zero += v != v ? v : 0.0F;
+      }
+      if (zero != zero)
+        return zero;
+    }
+  }
   double sum = 0.0;
 #pragma unroll 1
-  for (int k = 0; k < p.taps; ++k)
+  for (int k = 0; k < taps; ++k) {
+    const int t = t0 + k * dilation;
+    const bool inside = t >= 0 && t < p.len_in;
 #pragma unroll 1
-    for (int j = 0; j < p.cin && sum == sum; ++j) {
-      int c = j, t = m + p.first[phase] + k * p.dilation;
-      if (p.view_kernel != 0) {
-        c = j / p.view_kernel;
-        t = m * p.view_stride + p.first[0] + j % p.view_kernel;
-      }
+    for (int c = 0; c < channels && sum == sum; ++c) {
       float v = 0.0F;
-      if (t >= 0 && t < p.len_in) {
+      if (inside) {
         v = x[static_cast<size_t>(c) * p.len_in + t];
         if (p.alpha_in != nullptr)
           v = Snake(v, p.alpha_in[c], SnakeInverse(p.alpha_in[c]));
         if (p.in_act == kActElu)
           v = Elu(v);
       }
-      sum += static_cast<double>(v) * PackedWeight(p.w, p.w_rows, p.taps, p.cin,
-                                                   p.phases > 1 ? phase : batch, k, j, co);
+      sum += static_cast<double>(v) *
+             PackedWeight(p.w, p.w_rows, p.taps, p.cin, p.phases > 1 ? phase : batch,
+                          view ? 0 : k, view ? c * taps + k : c, co);
     }
+  }
   return static_cast<float>(sum);
 }
 
@@ -651,16 +674,16 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     __syncthreads();
     bool wide = false;
     // Four runs, and whether all of them are finite.
-    auto fours = [&](int q, floatx4* v) __attribute__((always_inline)) {
-      floatx4 zero = {0.0F, 0.0F, 0.0F, 0.0F};
+    auto run = [&](int q, int i) __attribute__((always_inline)) {
+      return *reinterpret_cast<const floatx4*>(
+          out + (mine - r0 + (4 * q + i) * kStride) * kRowFloats + tid % kRuns * 4);
+    };
+    auto check = [](floatx4 v, floatx4* zero) __attribute__((always_inline)) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[i] = *reinterpret_cast<const floatx4*>(
-            out + (mine - r0 + (4 * q + i) * kStride) * kRowFloats + tid % kRuns * 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          zero[e] = fmaf(v[i][e], 0.0F, zero[e]);
-      }
+      for (int e = 0; e < 4; ++e)
+        (*zero)[e] = fmaf(v[e], 0.0F, (*zero)[e]);
+    };
+    auto finite = [](floatx4 zero) __attribute__((always_inline)) {
       return (zero[0] + zero[1]) + (zero[2] + zero[3]) == 0.0F;
     };
 #pragma unroll 1
@@ -668,17 +691,28 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
       const Runs cur = next;
       if (q + 1 < kPer)
         next = gather(mine + 4 * (q + 1) * kStride);
-      floatx4 sums[4];
-      const bool finite = fours(q, sums);
-      wide |= !finite;
-      if (!UP && __builtin_expect(!finite, 0))  // y may be the residual
-        continue;
+      // Four runs are left out where one is not finite, since y may be the
+      // residual; phases have none, and none to leave out.
+      floatx4 sums[4], zero = {0.0F, 0.0F, 0.0F, 0.0F};
+      if (!UP) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sums[i] = run(q, i);
+          check(sums[i], &zero);
+        }
+        if (__builtin_expect(!finite(zero), 0)) {
+          wide = true;
+          continue;
+        }
+      }
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int local = mine + (4 * q + i) * kStride;
         if (co0 + local >= p.cout || n <= 0)
           continue;
-        floatx4 v = sums[i];
+        floatx4 v = UP ? run(q, i) : sums[i];
+        if (UP)
+          check(v, &zero);
         const size_t to = static_cast<size_t>(co0 + local) * p.len_out + at0;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -706,14 +740,19 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
               y_act[to + e] = v[e];
         }
       }
+      if (UP)
+        wide |= !finite(zero);
     }
     // The sums that are not finite are formed again, and their fours finished.
     if (__builtin_expect(wide, 0)) {
       const ConvParams& wp = ParamsAgain<ConvParams>();
 #pragma unroll 1
       for (int q = 0; q < kPer; ++q) {
-        floatx4 sums[4];
-        if (fours(q, sums))
+        floatx4 zero = {0.0F, 0.0F, 0.0F, 0.0F};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          check(run(q, i), &zero);
+        if (finite(zero))
           continue;
 #pragma unroll 1
         for (int k = 0; k < 16; ++k) {

@@ -235,6 +235,26 @@ def test_conv1d_of_the_largest_values(cin, cout, length, kernel, stride, groups,
         _finite_and_close(y.cpu().numpy(), want, size)
 
 
+@pytest.mark.parametrize("cin,cout,length,kernel,stride,split", [
+    (40, 33, 300, 1, 1, 0), (300, 130, 40, 1, 1, 1 << 20), (300, 70, 30, 7, 1, 1 << 20),
+    (40, 130, 211, 3, 2, 0), (70, 20, 90, 8, 4, 1 << 20)])
+def test_strided_and_split_conv1d_keep_infinities(cin, cout, length, kernel, stride, split):
+    """Infinite and NaN inputs give what 64 bits give, in the outputs that they reach only."""
+    rng = np.random.default_rng(cin + kernel)
+    x = rng.standard_normal((cin, length)).astype(np.float32)
+    x[3, 9], x[17, 20], x[20, 20], x[5, 27] = np.inf, np.inf, -np.inf, np.nan
+    w = rng.standard_normal((cout, cin, kernel)).astype(np.float32)
+    b = np.zeros(cout, np.float32)
+    with np.errstate(invalid="ignore"):
+        want = conv_exact(x, w, b, 1, stride, (kernel - 1) // 2)
+    y = dev(np.zeros(want.shape))
+    ov.op_conv1d_strided(dev(x), w, b, y, 1, stride, (kernel - 1) // 2, split_floats=split)
+    got, finite = y.cpu().numpy(), np.isfinite(want)
+    assert (np.isfinite(got) == finite).all()
+    np.testing.assert_array_equal(got[~finite], want[~finite].astype(np.float32))
+    np.testing.assert_allclose(got[finite], want[finite], rtol=1e-4, atol=1e-4)
+
+
 def test_conv1d_of_the_smallest_values():
     """Inputs around 2^-118, whose low parts are below bf16's least value 2^-133, against 64
     bits: each is kept to half of that, beside the tile edges' bound."""

@@ -7,7 +7,7 @@
 // bf16 parts (split.hpp). Bias, activations and the residual addition are
 // applied in the epilogue, straight from the accumulators. The sums are
 // nearer to the exact ones than the float32 matrix cores' (the decoder's
-// audio 1.2-2.1e-6 from 64 bits where those gave 1.9-4.6e-6).
+// audio 1.2-2.3e-6 from 64 bits where those gave 1.9-4.6e-6).
 #include "codec.hpp"
 #include "common.hpp"
 #include "kernels.hpp"
@@ -224,16 +224,17 @@ constexpr int TileChunk(int taps, int columns) {
 // VIEW reads the input through a strided window: K index j is tap j %
 // view_kernel of channel j / view_kernel (an im2col that is never stored).
 //
-// Bound by the matrix cores (their pipes 52-60 % busy at the 1.9 GHz this
-// work draws) at 128 channels and more; at 32 and 64 by them, the activations'
-// vector work and memory alike. At a 60 s signal: the k7 convolutions of 256
-// and 512 channels 200 TFLOP/s of float32 products (87 on the float32 matrix
-// cores), a residual unit of 128 / 64 / 32 channels 399 / 272 / 282 us where
-// its two launches took 492 / 329 / 397, the transposed convolutions 204 us
-// a launch where one phase per work-group, its outputs scattered, took 295.
+// Bound by the matrix cores (their pipes 58-69 % busy at the 1.9 GHz this
+// work draws) at 128 channels and more; at 32 and 64 (27 and 41 %) by them,
+// the activations' vector work and memory alike. At a 60 s signal: the k7
+// convolutions of 256 and 512 channels 195 TFLOP/s of float32 products (87 on
+// the float32 matrix cores), a residual unit of 128 / 64 / 32 channels 403 /
+// 268 / 280 us where its two launches took 492 / 329 / 397, the transposed
+// convolutions 202 us a launch where one phase per work-group, its outputs
+// scattered, took 295.
 // Splitting a chunk between its predecessor's products instead of before its
 // own: one-tap layers of 768 to 3072 channels at 500 positions 22.3 -> 20.6
-// and 28.8 -> 25.0 us, the transposed convolutions 230 -> 204 us.
+// and 28.8 -> 25.0 us, the transposed convolutions 230 -> 204 us a launch.
 enum ConvKind : int { kPlain, kView, kFused, kUp };
 
 template <int WM, int WN, int NT, int TAPS, int BUFS, ConvKind KIND>

@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void ConvKernel(ConvParams p) {
     group[q] = u / width;
     const int m = m0 + u % width;
     if (VIEW) {
-      at[q] = m * p.view_stride + lo;
+      at[q] = min(m, p.positions - 1) * p.view_stride + lo;  // columns past the last: not stored
     } else {
       const int t = m + lo;
 #pragma unroll
@@ -1092,7 +1092,7 @@ void LaunchConv(const ConvParams& params, hipStream_t stream) {
     Require(p.taps == 1 && p.phases == 1, "conv: a view has one tap and phase");
     Require(p.view_kernel >= 1 && p.view_stride >= 1 && p.channels >= 1 &&
                 static_cast<int64_t>(p.channels) * p.view_kernel == p.cin &&
-                (p.positions + int64_t{256}) * p.view_stride + p.view_kernel <
+                (p.positions - int64_t{1}) * p.view_stride + p.view_kernel <
                     (std::int64_t{1} << 31),
             "conv: bad view");
     DispatchTaps<1, kView>(p, stream);
